@@ -18,7 +18,10 @@
 #include <algorithm>
 #include <climits>
 #include <cstdlib>
+#include <cstring>
 #include <type_traits>
+
+extern "C" char** environ;
 
 namespace csahca {
 namespace {
@@ -513,6 +516,23 @@ __device__ __forceinline__ uint4 dequant8_bf16(uint2 w, uint32_t sbyte) {
     const uint32_t b1 = (word >> (16 * (i & 1) + 8)) & 0xffu;
     o[i] = static_cast<uint32_t>(float_to_bf16_bits(e4m3_to_f32(b0) * s)) |
            (static_cast<uint32_t>(float_to_bf16_bits(e4m3_to_f32(b1) * s)) << 16);
+  }
+  return make_uint4(o[0], o[1], o[2], o[3]);
+}
+
+// Eight codes by way of fp32 (exact e4m3 values, an fp32 product, round to
+// nearest even): the software decode's results for every scale byte, in 16
+// instructions.
+__device__ __forceinline__ uint4 dequant8_bf16_f32(uint2 w, uint32_t sbyte) {
+  typedef float f32x2_v __attribute__((ext_vector_type(2)));
+  const float s = ue8m0_to_f32(sbyte);
+  uint32_t o[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int word = static_cast<int>(i < 2 ? w.x : w.y);
+    const f32x2_v v = (i & 1) ? __builtin_amdgcn_cvt_pk_f32_fp8(word, true) : __builtin_amdgcn_cvt_pk_f32_fp8(word, false);
+    const bf16x2_t b = {static_cast<__bf16>(v[0] * s), static_cast<__bf16>(v[1] * s)};
+    o[i] = bf16x2_bits(b);
   }
   return make_uint4(o[0], o[1], o[2], o[3]);
 }
@@ -1536,6 +1556,524 @@ __global__ __launch_bounds__(NW * kWave) void dsv4_onepass_kernel(const int32_t*
   }
 }
 
+// ---------------------------------------------------------------------------
+// Wide kernel (dsv4_wide_kernel): one workgroup of 4 wavefronts = (query, 64
+// heads) and the query's whole slot list, walked in rounds of 64 slots, so a
+// row is fetched and dequantised once for 64 heads.
+//   * Loads: each wavefront takes 16 of a round's rows; a register is requested
+//     again (for the round after next) as soon as its chunk is dequantised into
+//     the next round's [slot][dim] bf16 tile in LDS, so a full round is always
+//     in flight.
+//   * QK: wavefront w scores 32 heads (half w % 2, the query operand resident
+//     in registers) against 32 slots (half w / 2) with
+//     v_mfma_f32_32x32x16_bf16: S^T[slot][head], lane l = head l % 32; the
+//     addresses of the rows two rounds on are formed between the MFMAs.
+//   * Softmax against a fixed reference: the maximum m of the first round.
+//     p = 2^(x - m) may exceed 1 later on; fp32 and bf16 hold it at the same
+//     relative precision up to 2^127, so the accumulators are never rescaled
+//     and no branch surrounds them (a rescale under a branch moved all 128 out
+//     of the registers the MFMAs use and back, every round).  Where a later
+//     score exceeds m by more than 2^64, or by more than 2^8 and an
+//     accumulator is not finite, the list is walked once more against the
+//     true maximum, which the first walk has found.
+//   * PV: wavefront w accumulates O^T for dims 128 w .. 128 w + 127 of all 64
+//     heads, V^T through ds_read_b64_tr_b16, P^T rows from LDS; half a chunk of
+//     the next tile is dequantised after every two MFMAs (left to itself the
+//     compiler ran the MFMAs and the conversions one after the other).
+// 64 heads of 512 fp32 sums and the bf16 query operand fill 256 of the 512
+// registers of a lane at one wavefront per SIMD; the tiles (two of 64 slots)
+// and P fill 146 KiB of LDS.  What bounds it: HBM at 256 queries (130 MB in
+// 39.5 us with 640 slots, 3.3 TB/s; the per-query kernel took 138.5 us), and
+// below that its serial chain, ~2.05 us a round (QK 0.7, softmax 0.3, PV 1.0)
+// and ~8 us around the rounds (query rows, first rows, output).
+// MFMA layouts (32x32x16): A lane l elem j = A[l%32][8(l/32)+j], B lane l elem
+// j = B[8(l/32)+j][l%32], C lane l elem i = C[8(i/4)+4(l/32)+i%4][l%32].
+// ---------------------------------------------------------------------------
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+constexpr int kWideHeads = 64;
+constexpr int kWideSlots = 64;
+constexpr int kWideWaves = 4;
+constexpr int kWidePRow = kWideSlots + 8;  // P row stride in bf16: 36 dwords, 16 rows on distinct 4-bank groups
+constexpr int kWideTile = kWideSlots * kQRow;  // bf16 of one K tile
+
+struct WideShared {
+  uint16_t tile[2][kWideTile];
+  uint16_t p[kWideHeads * kWidePRow];
+  float mx[2][kWideHeads];        // per slot half: maxima, then sums
+  float m[kWideHeads];            // the reference maxima
+  uint8_t ok[2][kWideSlots];      // per tile: the slot holds a row
+  uint32_t full[2][kWideWaves];   // per tile and loading wavefront: all its 16 slots do
+  uint32_t flag[kWideWaves];
+};
+static_assert(sizeof(WideShared) <= 160 * 1024, "LDS of one workgroup");
+
+// A cache as the wide kernel addresses it (pages below 2^31 bytes; others take
+// the other kernels).  A token's page is loc / page_size, formed as (loc *
+// magic) >> shift, so no branch between a division and a shift ends the block
+// of MFMAs it is computed among.
+struct WideView {
+  const uint8_t* base;
+  uint32_t num_pages, bpp, scale_off, page_size, magic, shift;
+};
+
+bool wide_view_fits(const CacheView& c) { return c.bpp < (int64_t{1} << 31); }
+
+WideView wide_view(const CacheView& c) {
+  // L = ceil(log2(page_size)), magic = ceil(2^(31+L) / page_size) < 2^32: its
+  // excess over the quotient is below 1, so for loc < 2^31 the product is off
+  // by less than 2^31 <= 2^(31+L) / page_size and the shift is exact.
+  const uint64_t d = static_cast<uint64_t>(std::max(c.page_size, 1));
+  uint32_t L = 0;
+  while ((uint64_t{1} << L) < d) ++L;
+  const uint64_t num = uint64_t{1} << (31 + L);
+  return WideView{c.base, static_cast<uint32_t>(std::min<int64_t>(c.num_pages, int64_t{1} << 31)),
+                  static_cast<uint32_t>(c.bpp), static_cast<uint32_t>(static_cast<uint64_t>(c.page_size) * kRowBytes),
+                  static_cast<uint32_t>(c.page_size), static_cast<uint32_t>((num + d - 1) / d), 31 + L};
+}
+
+struct WideArgs {
+  WideView swa, extra;
+  const float* sink;  // [heads] or null
+  bf16* out;
+  float qscale;
+};
+
+// 16 bytes at a constant offset from a row address (an immediate of the load).
+__device__ __forceinline__ uint4 load_at(const uint8_t* p, int off) {
+  const u32x4_t v = *reinterpret_cast<const __attribute__((address_space(1))) u32x4_t*>(
+      reinterpret_cast<uint64_t>(p) + static_cast<uint64_t>(off));
+  return make_uint4(v[0], v[1], v[2], v[3]);
+}
+__device__ __forceinline__ uint2 load8_at(const uint8_t* p) {
+  const u32x2_t v = *reinterpret_cast<const __attribute__((address_space(1))) u32x2_t*>(reinterpret_cast<uint64_t>(p));
+  return make_uint2(v[0], v[1]);
+}
+
+__global__ __launch_bounds__(kWideWaves * kWave, 1) void dsv4_wide_kernel(const int32_t* idx, const int32_t* eidx,
+                                                                          const int32_t* lens, const int32_t* elens,
+                                                                          int32_t topk_slots, int32_t extra_slots,
+                                                                          int32_t groups, int32_t nq, int32_t heads,
+                                                                          const bf16* __restrict__ q, WideArgs a) {
+  // (leading scalars: preloaded into SGPRs, as in the one-pass kernel)
+  __shared__ __align__(16) WideShared sm;
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int lane = tid % kWave;
+  const int grp = lane / 16, l16 = lane % 16;
+  const int hl = lane / 32, l32 = lane % 32;
+  const int hh = wave & 1, sb = wave >> 1;  // QK: head half, slot half
+  const uint32_t blk = blockIdx.x;
+  const uint32_t row8 = blk / 8;
+  const uint32_t gx = static_cast<uint32_t>(groups);
+  const int hg = static_cast<int>(row8 % gx);
+  const int64_t query = static_cast<int64_t>(row8 / gx) * 8 + blk % 8;
+  if (query >= nq) return;
+  const int h0 = hg * kWideHeads;
+  const int nh = min(kWideHeads, heads - h0);
+
+  // The query rows (whole rows per load; heads past the last repeat it, their
+  // results are dropped) and the sink, requested before anything waits.
+  const bf16* qrows = q + (query * heads + h0) * kDim + 8 * lane;
+  uint4 qs[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) qs[i] = load_global_u4(qrows + min(16 * wave + i, nh - 1) * kDim);
+  const float sink_raw = load_global_raw<float>(a.sink ? static_cast<const void*>(a.sink + h0 + min(lane, nh - 1))
+                                                       : static_cast<const void*>(q));
+  const int n_swa = lens ? max(0, min(lens[query], topk_slots)) : topk_slots;
+  const int n_extra = extra_slots > 0 ? (elens ? max(0, min(elens[query], extra_slots)) : extra_slots) : 0;
+  // The valid parts of the two lists as sub-tiles of 16 slots, one list after
+  // the other; sub-tile 4 r + w is wavefront w's of round r, so all the slots
+  // a wavefront loads in a round are of one list.
+  const int nsw = (n_swa + 15) >> 4, nsub = nsw + ((n_extra + 15) >> 4);
+  const int rounds = (nsub + 3) >> 2;
+
+  // Loading a round: lane (r8, c8) takes rows r8 and r8 + 8 of its wavefront's
+  // 16, so 8 lanes read 128 consecutive bytes of a row: chunks c8 + 8 j (j =
+  // 0..3) of 16 bytes of both (0..27 e4m3, 28..35 rope), and chunk 32 + c8 % 4
+  // of the first (c8 < 4) or the second.  (4 lanes a row: 64 bytes a row per
+  // load, was 10% slower at the memory-bound sizes.)
+  const int r8 = lane >> 3, c8 = lane & 7;
+  const bool hi4 = c8 >= 4;
+  struct Sub {
+    bool swa, live;
+    int j0, n;
+  };
+  auto sub_of = [&](int r) -> Sub {
+    const int u0 = 4 * r + wave, u = min(u0, nsub - 1);
+    const bool in = u < nsw;
+    return Sub{in, u0 < nsub, 16 * (in ? u : u - nsw), in ? n_swa : n_extra};
+  };
+  auto idx_issue = [&](int r, int32_t (&loc)[2]) {
+    const Sub s = sub_of(r);
+    const int32_t* list = s.swa ? idx + query * topk_slots : eidx + query * extra_slots;
+#pragma unroll
+    for (int rr = 0; rr < 2; ++rr) loc[rr] = list[min(s.j0 + r8 + 8 * rr, s.n - 1)];
+  };
+  struct Rows {
+    const uint8_t* row[2];    // at this lane's first chunk
+    const uint8_t* scale[2];
+    const uint8_t* tail;
+    bool ok[2];
+  };
+  // Absent and invalid slots read the zero row.  (Named here, outside the
+  // lambdas: a device variable named in one gets external linkage, and every
+  // kernel that uses it a load of its address.)
+  const uint64_t zero_row = reinterpret_cast<uint64_t>(g_dsv4_zero_row);
+  // The rows of a round from its slots' indices, in seven stages of about a
+  // dozen instructions (the main loop runs them between MFMAs).
+  struct RowMath {
+    WideView v;
+    int j0, nn;
+    uint32_t page[2], in_page[2];
+    uint64_t pg[2], row[2], scale[2];
+  };
+  auto rows_stage = [&](int stage, int r, const int32_t (&loc)[2], RowMath& x, Rows& w) {
+    if (stage == 0) {
+      const Sub s = sub_of(r);
+      x.v.base = s.swa ? a.swa.base : a.extra.base;
+      x.v.num_pages = s.swa ? a.swa.num_pages : a.extra.num_pages;
+      x.v.bpp = s.swa ? a.swa.bpp : a.extra.bpp;
+      x.v.scale_off = s.swa ? a.swa.scale_off : a.extra.scale_off;
+      x.v.page_size = s.swa ? a.swa.page_size : a.extra.page_size;
+      x.v.magic = s.swa ? a.swa.magic : a.extra.magic;
+      x.v.shift = s.swa ? a.swa.shift : a.extra.shift;
+      x.j0 = s.j0;
+      x.nn = s.live ? s.n : 0;
+    }
+    const int rr = (stage - 1) & 1;
+    if (stage == 1 || stage == 2) {
+      const uint32_t u = static_cast<uint32_t>(loc[rr]);
+      x.page[rr] = static_cast<uint32_t>((static_cast<uint64_t>(u) * x.v.magic) >> x.v.shift);
+      x.in_page[rr] = u - x.page[rr] * x.v.page_size;
+    }
+    if (stage == 3 || stage == 4) {
+      const uint64_t pg = static_cast<uint64_t>(x.page[rr]) * x.v.bpp + reinterpret_cast<uint64_t>(x.v.base);
+      x.row[rr] = static_cast<uint64_t>(x.in_page[rr]) * kRowBytes + pg;
+      x.scale[rr] = static_cast<uint64_t>(x.in_page[rr]) * kScaleBytes + (pg + x.v.scale_off);
+    }
+    if (stage == 5 || stage == 6) {
+      const bool ok = (x.j0 + r8 + 8 * rr < x.nn) && loc[rr] >= 0 && x.page[rr] < x.v.num_pages;
+      uint64_t row = ok ? x.row[rr] : zero_row, scale = ok ? x.scale[rr] : zero_row;
+      asm("" : "+v"(row), "+v"(scale));  // (keeps the choice a select; not volatile, so it may sit between MFMAs)
+      x.row[rr] = row;
+      w.ok[rr] = ok;
+      w.row[rr] = reinterpret_cast<const uint8_t*>(row + 16 * c8);
+      w.scale[rr] = reinterpret_cast<const uint8_t*>(scale);
+    }
+    if (stage == 6) {
+      // (bit masks: a choice between two array elements goes through the stack)
+      const uint64_t pick = hi4 ? ~uint64_t{0} : uint64_t{0};
+      w.tail = reinterpret_cast<const uint8_t*>(((x.row[1] & pick) | (x.row[0] & ~pick)) + 512 + 16 * (c8 & 3));
+    }
+  };
+  auto rows_at = [&](int r, const int32_t (&loc)[2], Rows& w) {
+    RowMath x;
+#pragma unroll
+    for (int st = 0; st < 7; ++st) rows_stage(st, r, loc, x, w);
+  };
+  auto scale_load = [&](const Rows& w, int rr) -> uint2 { return load8_at(w.scale[rr]); };
+  auto chunk_load = [&](const Rows& w, int k) -> uint4 {
+    return k == 8 ? load_at(w.tail, 0) : load_at(w.row[k >> 2], 128 * (k & 3));
+  };
+  // Half `h` of chunk k (8 values), dequantised, into tile `b` (e4m3 chunk c
+  // has scale byte c / 4; the tail chunk is one half).
+  auto half_store = [&](const uint4& c, const uint2 (&sc)[2], int k, int h, int b, auto general) {
+    uint16_t* t0 = sm.tile[b] + (16 * wave + r8) * kQRow;
+    if (k == 8) {
+      *reinterpret_cast<uint4*>(t0 + (hi4 ? 8 * kQRow : 0) + kNope + 32 + 8 * (c8 & 3)) = c;
+      return;
+    }
+    const int rr = k >> 2, j = k & 3;
+    uint16_t* trow = t0 + rr * 8 * kQRow;
+    const uint32_t word = j < 2 ? sc[rr].x : sc[rr].y;
+    const uint32_t sbyte = (word >> (16 * (j & 1) + (j < 3 && hi4 ? 8 : 0))) & 0xffu;
+    const uint2 w = h ? make_uint2(c.z, c.w) : make_uint2(c.x, c.y);
+    uint4 v;
+    if constexpr (decltype(general)::value)
+      v = dequant8_bf16_f32(w, sbyte);
+    else
+      v = dequant8_bf16_hw(w, sbyte);
+    uint16_t* dst = trow + 16 * (c8 + 8 * j) + 8 * h;
+    if (j == 3) {
+      // Chunks 24..27 e4m3, 28..31 rope (8 values as they are; written twice).
+      // Word by word: a choice between two vectors goes through the stack.
+      v = make_uint4(hi4 ? c.x : v.x, hi4 ? c.y : v.y, hi4 ? c.z : v.z, hi4 ? c.w : v.w);
+      dst = hi4 ? trow + kNope + 8 * (c8 - 4) : dst;
+    }
+    *reinterpret_cast<uint4*>(dst) = v;
+  };
+  auto chunk_store = [&](const uint4& c, const uint2 (&sc)[2], int k, int b, auto general) {
+    half_store(c, sc, k, 0, b, general);
+    if (k < 8) half_store(c, sc, k, 1, b, general);
+  };
+  // Which slots of the stored rows hold one, and (rare: a scale byte of 255)
+  // their e4m3 chunks once more, through the general decode.
+  auto tile_finish = [&](const Rows& w, bool any255, int b) {
+    const bool full = __all(w.ok[0] && w.ok[1]);
+    if (lane == 0) sm.full[b][wave] = full ? 1u : 0u;
+    if (!full && c8 == 0) {
+      sm.ok[b][16 * wave + r8] = w.ok[0];
+      sm.ok[b][16 * wave + r8 + 8] = w.ok[1];
+    }
+    if (any255) {
+      uint2 sc[2] = {scale_load(w, 0), scale_load(w, 1)};
+#pragma unroll
+      for (int k = 0; k < 8; ++k) chunk_store(chunk_load(w, k), sc, k, b, std::true_type{});
+    }
+  };
+  // A row's scale bytes hold a 255: high bits of the bytes equal to it (the
+  // pad byte may count: no harm).
+  auto bytes_255 = [&](const uint2& sc) -> uint32_t {
+    return ((((sc.x & 0x7f7f7f7fu) + 0x01010101u) & sc.x) | (((sc.y & 0x7f7f7f7fu) + 0x01010101u) & sc.y)) & 0x80808080u;
+  };
+
+  f32x16_t o[2][4];  // O^T[dims 128 wave + 32 db ..][heads 32 hb + l32]
+  float m = -INFINITY, l = 0.f;  // head 32 hh + l32; l: this lane's slots only
+  uint4 qb[32];                  // query operand: head 32 hh + l32, dims 16 t + 8 hl .. +7 of step t
+  int32_t loc0[2], loc1[2];
+  if (rounds > 0) {
+    idx_issue(0, loc0);
+    idx_issue(1, loc1);
+    // The query rows go through tile 1, which is written again only after
+    // every wavefront has read its operand.
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      *reinterpret_cast<uint4*>(sm.tile[1] + (16 * wave + i) * kQRow + 8 * lane) = qs[i];
+  }
+  for (int pass = 0;; ++pass) {
+    float mrun = -INFINITY;  // this lane's largest score
+    l = 0.f;
+    if (rounds > 0) {
+      int32_t loc[2];
+      Rows at, nx;
+      uint4 c[9];
+      rows_at(0, loc0, at);
+      uint2 sc[2] = {scale_load(at, 0), scale_load(at, 1)};
+#pragma unroll
+      for (int k = 0; k < 9; ++k) c[k] = chunk_load(at, k);
+      idx_issue(2, loc);
+      rows_at(1, loc1, nx);
+      {
+        const bool any255 = __any((bytes_255(sc[0]) | bytes_255(sc[1])) != 0u);
+#pragma unroll
+        for (int k = 0; k < 9; ++k) {
+          chunk_store(c[k], sc, k, 0, std::false_type{});
+          c[k] = chunk_load(nx, k);
+          if (k == 3 || k == 7) sc[k >> 2] = scale_load(nx, k >> 2);
+        }
+        tile_finish(at, any255, 0);
+      }
+      at = nx;
+      lds_barrier();
+      if (pass == 0) {
+#pragma unroll
+        for (int t = 0; t < 32; ++t)
+          qb[t] = *reinterpret_cast<const uint4*>(sm.tile[1] + (32 * hh + l32) * kQRow + 16 * t + 8 * hl);
+        // Most of the operand in AGPRs, which the MFMAs read directly: 128 of
+        // them hold O, 16 S, so 28 of the 32 steps fit.
+#pragma unroll
+        for (int t = 0; t < 28; ++t) {
+          u32x4_t w = {qb[t].x, qb[t].y, qb[t].z, qb[t].w};
+          asm volatile("" : "+a"(w));
+          qb[t] = make_uint4(w[0], w[1], w[2], w[3]);
+        }
+      }
+#pragma unroll
+      for (int hb = 0; hb < 2; ++hb)
+#pragma unroll
+        for (int db = 0; db < 4; ++db)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) o[hb][db][i] = 0.f;
+      for (int r = 0; r < rounds; ++r) {
+        const int b = r & 1;
+        // ---- QK: S^T of 32 slots x 32 heads; between the MFMAs the
+        // addresses of the rows two rounds on and the indices of the next ----
+        const bool full = (sm.full[b][2 * sb] & sm.full[b][2 * sb + 1]) != 0u;
+        const uint16_t* krow = sm.tile[b] + (32 * sb + l32) * kQRow + 8 * hl;
+        f32x16_t s;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[i] = 0.f;
+        {
+          // Eight operands in flight, one stage of the row addresses per four MFMAs.
+          uint4 kr[32];
+          RowMath rm;
+          int32_t locn[2];
+#pragma unroll
+          for (int t = 0; t < 8; ++t) kr[t] = *reinterpret_cast<const uint4*>(krow + 16 * t);
+#pragma unroll
+          for (int g4 = 0; g4 < 8; ++g4) {
+#pragma unroll
+            for (int t = 4 * g4; t < 4 * g4 + 4; ++t) {
+              if (t + 8 < 32) kr[t + 8] = *reinterpret_cast<const uint4*>(krow + 16 * (t + 8));
+              s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, kr[t]),
+                                                          __builtin_bit_cast(bf16x8_t, qb[t]), s, 0, 0, 0);
+            }
+            if (g4 < 7) rows_stage(g4, r + 2, loc, rm, nx);
+            if (g4 == 7) idx_issue(r + 3, locn);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          loc[0] = locn[0];
+          loc[1] = locn[1];
+        }
+        float x[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) x[i] = s[i] * a.qscale;
+        if (__builtin_amdgcn_readfirstlane(full) == 0) {  // absent or invalid slots: -inf
+#pragma unroll
+          for (int w = 0; w < 2; ++w) {
+            const bool wf = sm.full[b][2 * sb + w] != 0u;
+#pragma unroll
+            for (int i = 8 * w; i < 8 * w + 8; ++i)
+              x[i] = (wf || sm.ok[b][32 * sb + 8 * (i / 4) + 4 * hl + i % 4]) ? x[i] : -INFINITY;
+          }
+        }
+        float mw = x[0];
+#pragma unroll
+        for (int i = 1; i < 15; i += 2) mw = fmaxf(fmaxf(mw, x[i]), x[i + 1]);
+        mw = fmaxf(mw, x[15]);
+        mrun = fmaxf(mrun, mw);
+        if (r == 0 && pass == 0) {  // the reference: the first round's maximum of each head
+          mw = fmaxf(mw, __uint_as_float(lane_xor<32>(__float_as_uint(mw), lane)));
+          if (hl == 0) sm.mx[sb][32 * hh + l32] = mw;
+          lds_barrier();
+          m = fmaxf(sm.mx[0][32 * hh + l32], sm.mx[1][32 * hh + l32]);
+        }
+        // ---- P rows: masked scores are -inf and give 0 (with no finite
+        // reference, against 0) ----
+        const float mu = m == -INFINITY ? 0.f : m;
+        uint16_t* prow = sm.p + (32 * hh + l32) * kWidePRow + 32 * sb + 4 * hl;
+        float lp[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < 16; i += 4) {
+          float p[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            p[e] = fast_exp2(x[i + e] - mu);
+            lp[e] += p[e];
+          }
+          *reinterpret_cast<uint2*>(prow + 2 * i) = make_uint2(bf16x2_nb(p[0], p[1]), bf16x2_nb(p[2], p[3]));
+        }
+        l += (lp[0] + lp[1]) + (lp[2] + lp[3]);
+        lds_barrier();  // P; every wavefront is past PV of the previous round
+        // ---- PV: 128 dims x 64 heads, and the next round's tile between the
+        // MFMAs (past the list: the zero row) ----
+        const uint16_t* vsrc = sm.tile[b] + (8 * hl + l16 / 4) * kQRow + 128 * wave + 16 * (grp & 1) + 4 * (l16 % 4);
+        const uint16_t* psrc = sm.p + l32 * kWidePRow + 8 * hl;
+        uint4 pb[2][2], vt[2][4];
+        auto p_read = [&](int t, int hb) {
+          pb[t & 1][hb] = *reinterpret_cast<const uint4*>(psrc + 32 * hb * kWidePRow + 16 * t);
+        };
+        auto v_read = [&](int t, int db) {
+          const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t*)(vsrc + 16 * t * kQRow + 32 * db));
+          const i16x4_t hi =
+              __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t*)(vsrc + (16 * t + 4) * kQRow + 32 * db));
+          const u32x2_t lw = __builtin_bit_cast(u32x2_t, lo), hw = __builtin_bit_cast(u32x2_t, hi);
+          vt[t & 1][db] = make_uint4(lw[0], lw[1], hw[0], hw[1]);
+        };
+#pragma unroll
+        for (int hb = 0; hb < 2; ++hb) p_read(0, hb);
+#pragma unroll
+        for (int db = 0; db < 4; ++db) v_read(0, db);
+        const uint32_t s255 = bytes_255(sc[0]) | bytes_255(sc[1]);
+        // One step per 32 dims of 16 slots: two MFMAs, the reads of the step
+        // four on, half a chunk of the next tile.
+#pragma unroll
+        for (int st = 0; st < 16; ++st) {
+          const int t = st >> 2, db = st & 3, k = st >> 1;
+          if (t < 3) {
+            if (db < 2) p_read(t + 1, db);
+            v_read(t + 1, db);
+          }
+#pragma unroll
+          for (int hb = 0; hb < 2; ++hb)
+            o[hb][db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, vt[t & 1][db]),
+                                                                __builtin_bit_cast(bf16x8_t, pb[t & 1][hb]), o[hb][db],
+                                                                0, 0, 0);
+          // Each register is requested again as soon as it is stored: a full
+          // round in flight, and no copy of a register that a load is to fill
+          // (the copy would wait for it).
+          half_store(c[k], sc, k, st & 1, b ^ 1, std::false_type{});
+          if (st & 1) c[k] = chunk_load(nx, k);
+          if (st == 7 || st == 15) sc[st >> 3] = scale_load(nx, st >> 3);
+          if (st == 15) {
+            half_store(c[8], sc, 8, 0, b ^ 1, std::false_type{});
+            c[8] = chunk_load(nx, 8);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        tile_finish(at, __any(s255 != 0u), b ^ 1);
+        at = nx;
+        lds_barrier();  // the next tile; P is free
+      }
+    }
+    // Sums and maxima of all heads.
+    l += __uint_as_float(lane_xor<32>(__float_as_uint(l), lane));
+    mrun = fmaxf(mrun, __uint_as_float(lane_xor<32>(__float_as_uint(mrun), lane)));
+    if (pass != 0) break;
+    if (hl == 0) {
+      sm.mx[sb][32 * hh + l32] = mrun;
+      if (sb == 0) sm.m[32 * hh + l32] = m;
+    }
+    lds_barrier();
+    mrun = fmaxf(sm.mx[0][32 * hh + l32], sm.mx[1][32 * hh + l32]);
+    const float top = fmaxf(sm.mx[0][lane], sm.mx[1][lane]), ref = sm.m[lane];  // of head `lane`
+    bool over = top > ref + 64.f;
+    if (__any(top > ref + 8.f)) {  // the same in every wavefront
+      float big = 0.f;
+#pragma unroll
+      for (int hb = 0; hb < 2; ++hb)
+#pragma unroll
+        for (int db = 0; db < 4; ++db)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) big = fmaxf(big, o[hb][db][i] == o[hb][db][i] ? fabsf(o[hb][db][i]) : INFINITY);
+      over = over || big == INFINITY;
+    }
+    const bool any_over = __any(over);
+    if (lane == 0) sm.flag[wave] = any_over ? 1u : 0u;
+    lds_barrier();
+    if (__builtin_amdgcn_readfirstlane(static_cast<int>(sm.flag[0] | sm.flag[1] | sm.flag[2] | sm.flag[3])) == 0)
+      break;  // workgroup-uniform; at most two passes
+    m = mrun;
+  }
+  if (hl == 0) {
+    sm.mx[sb][32 * hh + l32] = l;
+    if (sb == 0) sm.m[32 * hh + l32] = m;
+  }
+  lds_barrier();
+  // Normalise with the sink as a virtual token of logit sink[h] and value 0
+  // (as in the other kernels); the results go out through LDS as whole rows.
+#pragma unroll
+  for (int hb = 0; hb < 2; ++hb) {
+    const int h = 32 * hb + l32;
+    const float L = sm.mx[0][h] + sm.mx[1][h], M = sm.m[h];
+    const float sk = a.sink ? __shfl(sink_raw, h) * kLog2e : -INFINITY;
+    const float mx = L > 0.f ? fmaxf(sk, M) : sk;
+    const float w = (L > 0.f && mx != -INFINITY) ? fast_exp2(M - mx) : 0.f;
+    float Lt = w * (L > 0.f ? L : 0.f);
+    if (a.sink && mx != -INFINITY) Lt += fast_exp2(sk - mx);
+    const float sc = L != L ? __builtin_nanf("") : (Lt > 0.f ? w / Lt : 0.f);
+    uint16_t* orow = sm.tile[0] + h * kQRow + 128 * wave + 4 * hl;
+#pragma unroll
+    for (int db = 0; db < 4; ++db)
+#pragma unroll
+      for (int i = 0; i < 16; i += 4) {
+        float y[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[e] = rounds > 0 ? o[hb][db][i + e] * sc : 0.f;
+        *reinterpret_cast<uint2*>(orow + 32 * db + 2 * i) = make_uint2(bf16x2_nb(y[0], y[1]), bf16x2_nb(y[2], y[3]));
+      }
+  }
+  lds_barrier();
+  uint4 y[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) y[i] = *reinterpret_cast<const uint4*>(sm.tile[0] + (16 * wave + i) * kQRow + 8 * lane);
+  bf16* ob = a.out + (query * heads + h0 + 16 * wave) * kDim + 8 * lane;
+  const int nw = nh - 16 * wave;  // rows of this wavefront
+#pragma unroll
+  for (int i = 0; i < 16; ++i)
+    if (i < nw) *reinterpret_cast<uint4*>(ob + i * kDim) = y[i];
+}
+
 constexpr int kMergeThreads = kDim / 4;  // 4 output columns per thread
 constexpr int kMergeChunk = 1024;        // tile weights staged in LDS per pass
 constexpr int kMergeFastTiles = 16;      // tiles merged straight from registers
@@ -1686,9 +2224,20 @@ size_t ws_bytes(int64_t nq, int64_t heads, int64_t tiles) {
   return ((ml + 255) & ~size_t{255}) + static_cast<size_t>(nq * heads * tiles * kDim) * sizeof(float);
 }
 
+// A CSAHCA_DSV4_* switch, or null.  The environment is read per call, and most
+// calls run with none of the switches set: one walk of it (any_switch) then
+// stands for the seven look-ups of a call.
+bool any_switch() {
+  for (char** e = environ; e && *e; ++e)
+    if ((*e)[0] == 'C' && std::strncmp(*e, "CSAHCA_DSV4_", 12) == 0) return true;
+  return false;
+}
+thread_local bool t_switches = true;  // set by each entry point for its call
+const char* env_switch(const char* name) { return t_switches ? std::getenv(name) : nullptr; }
+
 // Workgroup target of the MFMA split (CSAHCA_DSV4_MFMA_WGS, read per call).
 int64_t mfma_target_wgs() {
-  const char* e = std::getenv("CSAHCA_DSV4_MFMA_WGS");
+  const char* e = env_switch("CSAHCA_DSV4_MFMA_WGS");
   const long v = e ? std::strtol(e, nullptr, 10) : 0;
   return v > 0 ? v : 256;
 }
@@ -1708,7 +2257,7 @@ void mfma_splits(int64_t nq, int64_t heads, int64_t total_slots, int64_t* splits
 
 // CSAHCA_DSV4_MFMA=0 keeps every call on the VALU kernels (read per call).
 bool mfma_enabled() {
-  const char* e = std::getenv("CSAHCA_DSV4_MFMA");
+  const char* e = env_switch("CSAHCA_DSV4_MFMA");
   return !(e && e[0] == '0');
 }
 
@@ -1722,7 +2271,7 @@ bool mfma_enabled() {
 // per-query against 8.8-9.5 split).
 // CSAHCA_DSV4_QUERY=0 / =1 forces the choice (read per call).
 bool use_query_kernel(int64_t nq, int64_t heads, int64_t total_slots) {
-  const char* e = std::getenv("CSAHCA_DSV4_QUERY");
+  const char* e = env_switch("CSAHCA_DSV4_QUERY");
   if (e && (e[0] == '0' || e[0] == '1')) return e[0] == '1';
   const int64_t groups = ceil_div(std::max<int64_t>(1, heads), kQHeads);
   return nq * groups >= 64 || (total_slots > kMfmaSlots && total_slots <= 8 * kQSub);
@@ -1735,7 +2284,7 @@ bool use_query_kernel(int64_t nq, int64_t heads, int64_t total_slots) {
 // rounds of 8, the second half empty, are no faster than three of 4).
 // CSAHCA_DSV4_QWAVES=4/8 forces either.
 int query_waves(int64_t total_slots) {
-  const char* e = std::getenv("CSAHCA_DSV4_QWAVES");
+  const char* e = env_switch("CSAHCA_DSV4_QWAVES");
   if (e && (e[0] == '4' || e[0] == '8') && e[1] == 0) return e[0] - '0';
   return total_slots <= 8 * kQSub ? 8 : 4;
 }
@@ -1744,7 +2293,7 @@ int query_waves(int64_t total_slots) {
 // share of the output dims: the most of 4, 2 and 1 at which the workgroups
 // still fit one per CU.  CSAHCA_DSV4_QPARTS=1/2/4 forces a count.
 int query_dim_parts(int64_t nq, int64_t groups) {
-  const char* e = std::getenv("CSAHCA_DSV4_QPARTS");
+  const char* e = env_switch("CSAHCA_DSV4_QPARTS");
   if (e && (e[0] == '1' || e[0] == '2' || e[0] == '4') && e[1] == 0) return e[0] - '0';
   const int ncu = device_cu_count();
   const int64_t base = ceil_div(nq, 8) * 8 * groups;
@@ -1757,18 +2306,46 @@ int query_dim_parts(int64_t nq, int64_t groups) {
 // and so does CSAHCA_DSV4_QUERY=0 / 1, which forces the split / per-query
 // kernel (both read per call).
 bool use_onepass(int64_t total_slots) {
-  const char* e = std::getenv("CSAHCA_DSV4_ONEPASS");
+  const char* e = env_switch("CSAHCA_DSV4_ONEPASS");
   if (e && e[0] == '0' && e[1] == 0) return false;
-  const char* f = std::getenv("CSAHCA_DSV4_QUERY");
+  const char* f = env_switch("CSAHCA_DSV4_QUERY");
   if (f && (f[0] == '0' || f[0] == '1')) return false;
   return total_slots > 0 && total_slots <= kOpMaxSlots;
+}
+
+// The wide kernel (64 heads and the whole list in one workgroup) takes a call
+// with more than 16 heads whose (query, 16 heads) pairs would need more than
+// one workgroup of the other kernels per CU: those fetch and dequantise every
+// row once per 16 heads and dim part, and run in waves of one workgroup per CU.
+// Measured per call (graph period, us, other kernel / wide), lists <= 256
+// slots against the one-pass kernel, pairs > CUs:
+//   H 64: nq 64 (256 pairs) 128 / 192 slots 13.1 / 14.9 against 13.1 / 15.5,
+//   nq 80 18.4 / 21.0 against 13.6 / 15.7, nq 256 44.4 / 54.2 against
+//   17.9 / 20.5; H 24: nq 128 12.9 / 14.9 against 13.4 / 15.7, nq 192
+//   18.5 / 21.5 against 14.4 / 16.6;
+// longer lists against the per-query kernel, pairs >= CUs / 2: H 64, 384 / 640
+// slots: nq 32 21.1 / 32.8 against 21.3 / 29.4, nq 64 23.2 / 35.2 against
+// 21.7 / 30.0, nq 256 89.1 / 138.5 against 28.5 / 39.5.  With 16 heads or
+// fewer three quarters of its MFMA work would be padding (nq 256, 192 slots
+// 15.7 against 17.6).
+// CSAHCA_DSV4_WIDE=0 / 1 forces the choice; CSAHCA_DSV4_QUERY=0 / 1, which
+// forces a kernel of the longer lists, turns it off (all read per call).
+bool use_wide(int64_t nq, int64_t heads, int64_t total_slots) {
+  if (total_slots <= 0) return false;
+  const char* e = env_switch("CSAHCA_DSV4_WIDE");
+  if (e && (e[0] == '0' || e[0] == '1') && e[1] == 0) return e[0] == '1';
+  const int ncu = device_cu_count();
+  const int64_t pairs = ceil_div(nq, 8) * 8 * ceil_div(heads, kQHeads);
+  if (heads <= kQHeads || ncu <= 0 || (total_slots <= kOpMaxSlots ? pairs <= ncu : 2 * pairs < ncu)) return false;
+  const char* f = env_switch("CSAHCA_DSV4_QUERY");
+  return !(f && (f[0] == '0' || f[0] == '1'));
 }
 
 // Dim parts of the one-pass kernel: 4 where the workgroups still fit one per
 // CU, else 2 (a part of all 512 dims would not fit the V tiles in LDS).
 // CSAHCA_DSV4_QPARTS=2/4 forces a count.
 int onepass_dim_parts(int64_t nq, int64_t groups) {
-  const char* e = std::getenv("CSAHCA_DSV4_QPARTS");
+  const char* e = env_switch("CSAHCA_DSV4_QPARTS");
   if (e && (e[0] == '2' || e[0] == '4') && e[1] == 0) return e[0] - '0';
   const int ncu = device_cu_count();
   const int64_t base = ceil_div(nq, 8) * 8 * groups;
@@ -1799,6 +2376,7 @@ int dsv4_run(const Dsv4Call& c) {
   if (c.nq == 0 || c.heads == 0) return CSAHCA_OK;
   CSAHCA_REQUIRE(c.q && c.out, "null tensor pointer");
   CSAHCA_REQUIRE(c.idx || c.topk_slots == 0 || c.nq == 0, "null token_indices pointer");
+  t_switches = any_switch();
   const int64_t total = c.topk_slots + c.extra_slots;
   CSAHCA_REQUIRE(total <= INT_MAX && c.nq <= INT_MAX && c.heads <= INT_MAX, "too many slots");
   const bool vec = reinterpret_cast<uintptr_t>(c.swa.base) % 16 == 0 && c.swa.bpp % 16 == 0 &&
@@ -1837,6 +2415,21 @@ int dsv4_run(const Dsv4Call& c) {
   a.num_tiles = static_cast<int>(tiles);
   a.qscale = static_cast<float>(c.softmax_scale) * kLog2e;
   hipStream_t stream = static_cast<hipStream_t>(c.stream);
+  if (use_mfma && reinterpret_cast<uintptr_t>(c.out) % 16 == 0 && use_wide(c.nq, c.heads, total) &&
+      wide_view_fits(c.swa) && (c.extra_slots == 0 || wide_view_fits(c.extra))) {
+    WideArgs wa;
+    wa.swa = wide_view(c.swa);
+    wa.extra = wide_view(c.extra);
+    wa.sink = c.sink;
+    wa.out = static_cast<bf16*>(c.out);
+    wa.qscale = a.qscale;
+    const int groups = static_cast<int>(ceil_div(c.heads, kWideHeads));
+    const int64_t blocks = ceil_div(c.nq, 8) * 8 * groups;  // query q's head groups x: blocks q%8 + 8 (x + G q/8)
+    CSAHCA_REQUIRE(blocks <= INT32_MAX, "too many DSV4 work items");
+    return launch("dsv4_wide_kernel", dsv4_wide_kernel, dim3(static_cast<uint32_t>(blocks)), dim3(kWideWaves * kWave),
+                  0, stream, a.idx, a.eidx, a.lens, a.elens, a.topk_slots, a.extra_slots, groups,
+                  static_cast<int32_t>(c.nq), a.heads, static_cast<const bf16*>(c.q), wa);
+  }
   if (use_mfma && reinterpret_cast<uintptr_t>(c.out) % 8 == 0 && use_onepass(total)) {
     QueryArgs qa;
     qa.nq = c.nq;
@@ -1850,7 +2443,7 @@ int dsv4_run(const Dsv4Call& c) {
     CSAHCA_REQUIRE(blocks <= INT32_MAX, "too many DSV4 work items");
     // 12 wavefronts with one sub-tile each for lists of up to 192 slots, else
     // 8 with two (CSAHCA_DSV4_OPWAVES=8 / 12 forces either where it fits).
-    const char* ew = std::getenv("CSAHCA_DSV4_OPWAVES");
+    const char* ew = env_switch("CSAHCA_DSV4_OPWAVES");
     const bool w12 = ew ? (std::atoi(ew) == 12 && total <= 12 * kQSub) : total <= 12 * kQSub;
     auto kfn = w12 ? (ds == 4 ? dsv4_onepass_kernel<12, 1, 4> : dsv4_onepass_kernel<12, 1, 2>)
                    : (ds == 4 ? dsv4_onepass_kernel<8, 2, 4> : dsv4_onepass_kernel<8, 2, 2>);
@@ -1934,6 +2527,7 @@ extern "C" size_t csahca_dsv4_decode_workspace_bytes(int64_t num_queries, int64_
                                                      int64_t topk_slots, int64_t extra_topk_slots,
                                                      int64_t tile_size) {
   if (num_queries < 0 || heads < 0 || topk_slots < 0 || extra_topk_slots < 0) return 0;
+  t_switches = any_switch();
   int64_t tile, tiles, splits, tps;
   dsv4_tiling(num_queries, heads, topk_slots + extra_topk_slots, tile_size, &tile, &tiles);
   mfma_splits(num_queries, heads, topk_slots + extra_topk_slots, &splits, &tps);

@@ -1,0 +1,142 @@
+"""The DSV4 kernel for many heads and queries (64 heads and the whole slot list
+in one workgroup) against the CPU oracle, at the edges of its tiles: 16-slot
+sub-tiles, 64-slot rounds, 64-head groups, odd pages.  CSAHCA_DSV4_WIDE=1 routes
+these small calls to it.  Tolerance: the FP8-cache bar |got - ref| <= 5e-2 +
+5e-2 |ref|, unless a test says otherwise."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from csahca_amd import extension, native
+from csahca_amd.dsv4_layout import pack_dsv4_cache
+from csahca_amd.synthetic import make_dsv4_case
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+SCALE = 1.0 / math.sqrt(512)
+
+
+@pytest.fixture(autouse=True)
+def _wide(monkeypatch):
+    if not torch.cuda.is_available():
+        pytest.fail("no HIP device visible")
+    native.lib()
+    monkeypatch.setenv("CSAHCA_DSV4_WIDE", "1")
+
+
+def gpu_out(c, sink=True):
+    d = lambda t: None if t is None else t.to(DEV)
+    s = d(c.attn_sink) if sink else None
+    if c.extra_cache is not None:
+        return extension.dsv4_sparse_decode_forward(d(c.q), d(c.cache), d(c.token_indices), d(c.topk_lengths),
+                                                    d(c.extra_cache), d(c.extra_token_indices),
+                                                    d(c.extra_topk_lengths), s, c.page_size, c.extra_page_size, SCALE)
+    return extension.dsv4_swa_decode_forward(d(c.q), d(c.cache), d(c.token_indices), d(c.topk_lengths), s,
+                                             c.page_size, SCALE)
+
+
+def oracle_out(c, sink=True):
+    kw = {}
+    if c.extra_cache is not None:
+        kw = dict(extra_cache=c.extra_cache.cpu(), extra_token_indices=c.extra_token_indices.cpu(),
+                  extra_topk_lengths=None if c.extra_topk_lengths is None else c.extra_topk_lengths.cpu(),
+                  extra_page_size=c.extra_page_size)
+    return oracle.dsv4_reference_attention(c.q.cpu(), c.cache.cpu(), c.token_indices.cpu(),
+                                           None if c.topk_lengths is None else c.topk_lengths.cpu(),
+                                           c.attn_sink.cpu() if sink else None, page_size=c.page_size,
+                                           softmax_scale=SCALE, **kw)
+
+
+def assert_close(got, ref, atol=5e-2, rtol=5e-2):
+    g = got.detach().double().cpu().numpy()
+    assert g.shape == ref.shape
+    assert np.array_equal(np.isnan(g), np.isnan(ref))
+    diff = np.abs(np.nan_to_num(g) - np.nan_to_num(ref))
+    bad = diff > atol + rtol * np.abs(np.nan_to_num(ref))
+    assert not bad.any(), f"max_abs={diff.max():.3e} bad={int(bad.sum())}/{bad.size}"
+
+
+@pytest.mark.parametrize("heads,top_k,extra_top_k,page,extra_page", [
+    (64, 1, 0, 64, 0),        # one slot
+    (17, 15, 0, 64, 0),       # less than a sub-tile; 17 of 64 heads
+    (64, 16, 1, 64, 16),      # a full sub-tile and one slot of the other list
+    (33, 17, 15, 48, 48),     # pages that are no power of two
+    (64, 63, 0, 1, 0),        # pages of one token
+    (65, 64, 64, 64, 16),     # whole rounds; a second head group of one head
+    (70, 65, 33, 64, 100),    # one slot into a round
+    (64, 128, 64, 256, 64),   # the window and its C4 entries
+    (24, 128, 512, 64, 1),    # ten rounds
+    (128, 100, 157, 64, 64),  # ragged in both lists
+])
+@pytest.mark.parametrize("lengths", ["full", "ragged", "none"])
+def test_wide_kernel_matches_oracle(heads, top_k, extra_top_k, page, extra_page, lengths):
+    c = make_dsv4_case(compress_ratio=4 if extra_top_k else 0, num_queries=9, heads=heads, num_tokens=700, top_k=top_k,
+                       page_size=page, extra_tokens=600, extra_top_k=extra_top_k, extra_page_size=extra_page or None,
+                       full_lengths=lengths == "full", seed=heads + top_k, device="cpu")
+    if lengths == "ragged":
+        c.topk_lengths[0] = 0                     # no window slots: the second list starts the first round
+        c.topk_lengths[1] = min(top_k, 5)
+        c.token_indices[2, 0] = -1
+        c.token_indices[3, :] = -1                # a whole list of skipped slots
+        if extra_top_k:
+            c.extra_topk_lengths[1] = 0
+            c.extra_topk_lengths[4] = 1
+            c.extra_token_indices[5, 0] = 10_000_000  # a page past the cache
+    elif lengths == "none":
+        c.topk_lengths = None
+        c.extra_topk_lengths = None
+    assert_close(gpu_out(c), oracle_out(c))
+    assert_close(gpu_out(c, sink=False), oracle_out(c, sink=False))
+
+
+@pytest.mark.parametrize("jump", [0.5, 40.0, 4000.0])
+def test_wide_kernel_scores_that_outgrow_the_first_round(jump):
+    """Probabilities are formed against the first round's maximum; later scores
+    that exceed it by up to 2^64 (jump 40: some tens of nats) are kept as they
+    are, larger ones (jump 4000) take the second walk.  Against the oracle and
+    against the other kernels, whose maximum moves."""
+    c = make_dsv4_case(compress_ratio=0, num_queries=5, heads=64, num_tokens=512, top_k=200, page_size=64,
+                       full_lengths=True, seed=3, pack=False, device="cpu")
+    c.token_indices = torch.arange(200, dtype=torch.int32).repeat(5, 1)
+    rows = c.k_tokens.float()
+    rows[:64] *= 0.01
+    rows[130:] *= jump
+    c.cache = pack_dsv4_cache(rows.to(torch.bfloat16), page_size=64)
+    ref = oracle_out(c)
+    # the outputs are of the rows' own magnitude: the bar relative to it
+    assert_close(gpu_out(c) / max(jump, 1.0), ref / max(jump, 1.0))
+
+
+def test_wide_kernel_scale_byte_255_poisons_its_query_only():
+    c = make_dsv4_case(compress_ratio=0, num_queries=4, heads=64, num_tokens=256, top_k=70, page_size=64,
+                       full_lengths=True, seed=8, device="cpu")
+    c.token_indices = (torch.arange(70, dtype=torch.int32)[None] + 64 * torch.arange(4, dtype=torch.int32)[:, None]) % 250
+    c.token_indices[:, :] = torch.where(c.token_indices == 200, 0, c.token_indices)
+    c.token_indices[2, 67] = 200  # only query 2 sees row 200
+    sb = 64 * 576 + (200 % 64) * 8
+    c.cache[200 // 64, sb + 3] = 255
+    ref = oracle_out(c)
+    assert np.isnan(ref[2]).all() and np.isfinite(ref[[0, 1, 3]]).all()
+    assert_close(gpu_out(c), ref)
+
+
+def test_wide_kernel_decodes_every_code_exactly():
+    """One valid slot and no sink: the output is the dequantised row, for every
+    finite e4m3 code under scale bytes over their range."""
+    scales = [0, 1, 90, 120, 127, 140, 200, 246]
+    cache = torch.zeros(8, 64 * 584 // 576 * 576 + 576, dtype=torch.uint8)
+    codes = torch.tensor([b for b in range(256) if b & 0x7F != 0x7F], dtype=torch.uint8)
+    for i, s in enumerate(scales):
+        cache[i, :448] = codes.roll(7 * i).repeat(2)[:448]
+        cache[i, 64 * 576:64 * 576 + 7] = s
+    q = torch.randn(8, 64, 512, generator=torch.Generator().manual_seed(0)).to(torch.bfloat16) * 1e-30
+    out = extension.dsv4_swa_decode_forward(q.to(DEV), cache.to(DEV),
+                                            (64 * torch.arange(8, dtype=torch.int32))[:, None].to(DEV), None, None, 64,
+                                            SCALE)
+    want = oracle.dsv4_reference_attention(q, cache, (64 * torch.arange(8, dtype=torch.int32))[:, None], None, None,
+                                           page_size=64, softmax_scale=SCALE)
+    got = out.double().cpu().numpy()
+    assert np.array_equal(got, torch.from_numpy(np.asarray(want)).to(torch.bfloat16).double().numpy())
