@@ -12,8 +12,9 @@
 //                        (b,h); K/V rows are fetched with 16-byte lane loads so
 //                        one wavefront-wide load moves whole rows; online
 //                        softmax in registers; fp32 partial (m, l, acc[D]).
-//   5. csa_merge_kernel: log-sum-exp merge of the partials of each (b,h), with
-//                        all partial loads independent of each other.
+//   5. csa_merge_*     : log-sum-exp merge of the partials of each (b,h) over 32
+//                        columns a workgroup, with all partial loads
+//                        independent of each other.
 // csa_step.hip fuses 2-5 into one launch.  All offsets are 64-bit.
 #include "csa_device.hpp"
 
@@ -190,114 +191,6 @@ __global__ __launch_bounds__(64) void csa_attend_generic_kernel(
   }
 }
 
-constexpr int kMergeRows = 64;  // partial rows per thread in the one-round-trip merge
-
-// Block-wide reductions for 256-thread blocks.
-__device__ __forceinline__ float block_max256(float v, float* red) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) v = fmaxf(v, xor_lanes(v, off));
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  v = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-  __syncthreads();
-  return v;
-}
-__device__ __forceinline__ float block_sum256(float v, float* red) {
-  v = wave_sum(v);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  v = (red[0] + red[1]) + (red[2] + red[3]);
-  __syncthreads();
-  return v;
-}
-
-// Log-sum-exp merge of the split partials of one (b,h) (the merge pass of
-// csrc/csa_attention.cu:224-274): M = max m_t, L = sum_{l_t>0} l_t 2^(m_t-M),
-// out = sum_{l_t>0} 2^(m_t-M) acc_t / L, or 0 when L is not positive.
-// 256 threads; the tile loops carry no data-dependent branches, so their loads
-// issue back to back.  Column d is summed by G = max(1, 256 / D) thread groups.
-template <typename T>
-__global__ __launch_bounds__(256) void csa_merge_kernel(const float* __restrict__ part_ml,
-                                                        const float* __restrict__ part_acc,
-                                                        T* __restrict__ out, int D, int num_tiles) {
-  __shared__ float red[4];
-  __shared__ float colsum[256];
-  __shared__ float wts[256];
-  const int64_t bh = blockIdx.x;
-  const float* ml = part_ml + 2 * bh * num_tiles;
-  const float* pa = part_acc + bh * num_tiles * static_cast<int64_t>(D);
-  const int tid = threadIdx.x;
-  if (D <= 256 && num_tiles <= 256 && num_tiles <= kMergeRows * (256 / D)) {
-    // One memory round trip: every thread requests its column of each of its
-    // partial rows and (m, l) of tile `tid` before anything waits; the tile
-    // weights then meet in LDS.
-    const int G = 256 / D, g = tid / D, d = tid - g * D;
-    float x[kMergeRows];
-#pragma unroll
-    for (int i = 0; i < kMergeRows; ++i) {
-      const int t = g + i * G;
-      x[i] = (g < G && t < num_tiles) ? pa[static_cast<int64_t>(t) * D + d] : 0.f;
-    }
-    const float mt = tid < num_tiles ? ml[2 * tid] : -INFINITY;
-    const float lt = tid < num_tiles ? ml[2 * tid + 1] : 0.f;
-    const float M = block_max256(lt > 0.f ? mt : -INFINITY, red);
-    const float w = (lt > 0.f && M != -INFINITY) ? fast_exp2(mt - M) : 0.f;
-    wts[tid] = w;
-    const float Lt = block_sum256(w * lt, red);  // its barriers also publish wts
-    float a = 0.f;
-#pragma unroll
-    for (int i = 0; i < kMergeRows; ++i) {
-      const int t = g + i * G;
-      if (g < G && t < num_tiles) a = fmaf(wts[t], x[i], a);
-    }
-    colsum[tid] = a;
-    __syncthreads();
-    if (tid < D) {
-      float o = 0.f;
-      for (int j = 0; j < G; ++j) o += colsum[j * D + tid];
-      out[bh * D + tid] = from_f32<T>(Lt > 0.f ? o / Lt : 0.f);
-    }
-    return;
-  }
-  float mx = -INFINITY;
-  for (int t = threadIdx.x; t < num_tiles; t += 256) mx = fmaxf(mx, ml[2 * t]);
-  mx = block_max256(mx, red);
-  float L = 0.f;
-  if (mx != -INFINITY) {
-    for (int t = threadIdx.x; t < num_tiles; t += 256) {
-      const float lt = ml[2 * t + 1];
-      L += lt > 0.f ? lt * fast_exp2(ml[2 * t] - mx) : 0.f;
-    }
-  }
-  L = block_sum256(L, red);
-  const float inv = (mx != -INFINITY && L > 0.f) ? 1.f / L : 0.f;
-  const int G = D >= 256 ? 1 : 256 / D;
-  const int g = threadIdx.x / (D >= 256 ? 256 : D);
-  for (int d0 = 0; d0 < D; d0 += (D >= 256 ? 256 : D)) {
-    const int d = d0 + threadIdx.x % (D >= 256 ? 256 : D);
-    float a = 0.f;
-    if (g < G && d < D && inv > 0.f) {
-#pragma unroll 8
-      for (int t = g; t < num_tiles; t += G) {
-        const float lt = ml[2 * t + 1];
-        const float w = lt > 0.f ? fast_exp2(ml[2 * t] - mx) : 0.f;
-        a = fmaf(w, pa[static_cast<int64_t>(t) * D + d], a);
-      }
-    }
-    if (G > 1) {
-      colsum[threadIdx.x] = a;
-      __syncthreads();
-      if (g == 0 && d < D) {
-        for (int j = 1; j < G; ++j) a += colsum[threadIdx.x + j * D];
-        out[bh * D + d] = from_f32<T>(a * inv);
-      }
-      __syncthreads();
-    } else if (d < D) {
-      out[bh * D + d] = from_f32<T>(a * inv);
-    }
-  }
-}
-
 // Merge of at most kMergeColTiles partials per head, spread over workgroups
 // of (head, kMergeCols output columns): 256 threads = kMergeCols columns x 8
 // tile groups.  Every load -- the thread's tiles of its column, and lane l's
@@ -350,6 +243,85 @@ __global__ __launch_bounds__(256) void csa_merge_cols_kernel(const float* __rest
 #pragma unroll
     for (int j = 0; j < kMergeGroups; ++j) o += colsum[j * kMergeCols + tid];
     out[bh * D + d] = from_f32<T>(L > 0.f ? o / L : 0.f);
+  }
+}
+
+// The same merge over any number of partials (split_tile gives more than
+// kMergeColTiles only to heads with long selections): the maximum over all
+// tiles first, then kMergePass tiles at a time -- weights once per workgroup
+// into LDS, then every thread its column of the pass's tiles g, g + 8, ...,
+// eight loads in flight.  (Whole op, before / after this merge and the split
+// rule, tile 8, D 128: B1 H1 65536 slots 1397 / 18.2 us, B1 H8 32768 slots
+// 770 / 32.1 us, 16384 slots 381 / 17.5 us; one workgroup per head summed all
+// columns, tile after tile.)
+constexpr int kMergePass = 1024;
+
+template <typename T>
+__global__ __launch_bounds__(256) void csa_merge_long_kernel(const float* __restrict__ part_ml,
+                                                             const float* __restrict__ part_acc,
+                                                             T* __restrict__ out, int D, int num_tiles,
+                                                             int col_blocks) {
+  __shared__ float wts[kMergePass];
+  __shared__ float red[4];
+  __shared__ float colsum[256];
+  const int tid = threadIdx.x;
+  const int64_t bh = blockIdx.x / col_blocks;
+  const int cb = static_cast<int>(blockIdx.x - bh * col_blocks);
+  const int cl = tid % kMergeCols, g = tid / kMergeCols;
+  const int d = cb * kMergeCols + cl;
+  const float* ml = part_ml + 2 * bh * num_tiles;
+  const float* pa = part_acc + bh * num_tiles * static_cast<int64_t>(D) + (d < D ? d : 0);
+  float M = -INFINITY;
+#pragma unroll 4
+  for (int t = tid; t < num_tiles; t += 256) {
+    const float2 v = *reinterpret_cast<const float2*>(ml + 2 * static_cast<int64_t>(t));
+    M = fmaxf(M, v.y > 0.f ? v.x : -INFINITY);
+  }
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) M = fmaxf(M, xor_lanes(M, off));
+  if (tid % kWave == 0) red[tid / kWave] = M;
+  __syncthreads();
+  M = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  float a = 0.f, L = 0.f;
+  for (int t0 = 0; t0 < num_tiles; t0 += kMergePass) {
+    const int n = min(kMergePass, num_tiles - t0);
+    __syncthreads();  // the previous pass's weights are read
+    for (int t = tid; t < kMergePass; t += 256) {
+      float w = 0.f;
+      if (t < n && M != -INFINITY) {
+        const float2 v = *reinterpret_cast<const float2*>(ml + 2 * static_cast<int64_t>(t0 + t));
+        w = v.y > 0.f ? fast_exp2(v.x - M) : 0.f;
+        L = fmaf(w, v.y > 0.f ? v.y : 0.f, L);
+      }
+      wts[t] = w;
+    }
+    __syncthreads();
+    const float* pt = pa + static_cast<int64_t>(t0) * D;
+    for (int t = g; t < n; t += 8 * kMergeGroups) {
+      float x[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {  // (tiles past the pass re-read tile t at weight 0)
+        const int ti = t + i * kMergeGroups;
+        x[i] = load_global_raw<float>(pt + static_cast<int64_t>(ti < n ? ti : t) * D);
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int ti = t + i * kMergeGroups;
+        a = fmaf(ti < n ? wts[ti] : 0.f, x[i], a);
+      }
+    }
+  }
+  L = wave_sum(L);
+  __syncthreads();
+  if (tid % kWave == 0) red[tid / kWave] = L;
+  colsum[tid] = a;
+  __syncthreads();
+  if (tid < kMergeCols && d < D) {
+    const float Lt = (red[0] + red[1]) + (red[2] + red[3]);
+    float o = 0.f;
+#pragma unroll
+    for (int j = 0; j < kMergeGroups; ++j) o += colsum[j * kMergeCols + tid];
+    out[bh * D + d] = from_f32<T>(Lt > 0.f ? o / Lt : 0.f);
   }
 }
 
@@ -525,6 +497,29 @@ size_t decode_ws_bytes(int64_t bh, int64_t D, int64_t tiles) {
   return ml_al + static_cast<size_t>(bh * tiles * D) * sizeof(float);
 }
 
+// Slots per wavefront of the split: the caller's tile, or the smallest multiple
+// of it that
+//   * fills one batch of row loads of the attend kernel (16 slots at 16-bit
+//     head_dim 128, 32 at 64, 4 in the generic kernel; a smaller tile re-reads
+//     its last row);
+//   * leaves a head at most 64 tiles, the one-round-trip merge, as long as that
+//     makes tiles of at most 128 slots;
+//   * leaves the call at most 8192 wavefronts (32 per CU): more only write and
+//     merge more partials.
+// A tile is a hint for the split, and the partials of several of the caller's
+// tiles are one partial of their union, so the workspace the caller sized for
+// its own tile holds them.  Measured (graph period, us, tile 8 as called /
+// split chosen): B1 H8 D128 top-8 5.31 / 5.06, top-32 49.3 / 7.3; B8 top-16
+// 16.4 / 10.3, top-32 60.6 / 15.3; B32 top-32 104.7 / 56.7; B4 H12 D64 f16
+// 480 slots 7.3 / 6.4; f32 D256 512 slots 9.4 (kept at 8).
+int64_t split_tile(int64_t tile, int64_t total, int64_t bh, int64_t D, int64_t esz) {
+  const bool vec = (D == 64 || D == 128 || D == 256 || D == 512) && D * esz / 16 <= kWave;
+  const int64_t batch = vec ? 4 * (kWave / (D * esz / 16)) : 4;
+  const int64_t want = std::max({batch, std::min<int64_t>(ceil_div(total, kMergeColTiles), 128), ceil_div(total * bh, 8192)});
+  const int64_t t = tile >= want ? tile : ceil_div(want, tile) * tile;
+  return std::min<int64_t>(t, std::max<int64_t>(total, 1));
+}
+
 template <typename T, typename IdxT>
 int launch_attend(const void* q, const void* k, const void* v, const void* idx, float* part_ml,
                   float* part_acc, int64_t bh, int64_t S, int64_t D, int top_k, int chunk,
@@ -585,16 +580,19 @@ int csa_decode_impl(const void* q, const void* k, const void* v, const void* idx
   if (bh == 0 || D == 0) return CSAHCA_OK;
   CSAHCA_REQUIRE(q && out && (S == 0 || (k && v)) && (idx || top_k == 0), "null tensor pointer");
   const int64_t total = top_k * chunk;
-  const int64_t tiles = std::max<int64_t>(1, ceil_div(total, tile));
-  CSAHCA_REQUIRE(bh * tiles <= INT32_MAX, "too many split-KV work items");
-  const size_t need = decode_ws_bytes(bh, D, tiles);
+  const int64_t asked = std::max<int64_t>(1, ceil_div(total, tile));
+  CSAHCA_REQUIRE(bh * asked <= INT32_MAX, "too many split-KV work items");
+  const size_t need = decode_ws_bytes(bh, D, asked);
   if (workspace == nullptr || workspace_bytes < need)
     return fail(CSAHCA_ERR_WORKSPACE, "workspace too small for csa decode");
+  const int64_t esz = dtype == CSAHCA_F64 ? 8 : dtype == CSAHCA_F32 ? 4 : 2;
+  tile = split_tile(tile, total, bh, D, esz);
+  const int64_t tiles = std::max<int64_t>(1, ceil_div(total, tile));  // <= asked
   float* part_ml = static_cast<float*>(workspace);
   const size_t ml = static_cast<size_t>(bh * tiles * 2) * sizeof(float);
   float* part_acc = reinterpret_cast<float*>(static_cast<char*>(workspace) + ((ml + 255) & ~size_t{255}));
   hipStream_t stream = static_cast<hipStream_t>(stream_ptr);
-  const int tl = static_cast<int>(std::min<int64_t>(tile, std::max<int64_t>(total, 1)));
+  const int tl = static_cast<int>(tile);
   // Stand-ins for pointers that are never dereferenced (no selected slots / no tokens).
   const void* idx_ok = idx ? idx : q;
   const void* k_ok = k ? k : q;
@@ -615,9 +613,11 @@ int csa_decode_impl(const void* q, const void* k, const void* v, const void* idx
                     dim3(256), 0, stream, static_cast<const float*>(part_ml), static_cast<const float*>(part_acc),
                     static_cast<T*>(out), static_cast<int>(D), static_cast<int>(tiles), static_cast<int>(cbs));
     }
-    return launch("csa_merge_kernel", csa_merge_kernel<T>, dim3(static_cast<uint32_t>(bh)), dim3(256), 0,
-                  stream, static_cast<const float*>(part_ml), static_cast<const float*>(part_acc),
-                  static_cast<T*>(out), static_cast<int>(D), static_cast<int>(tiles));
+    const int64_t cbs = ceil_div(D, kMergeCols);
+    CSAHCA_REQUIRE(bh * cbs <= INT32_MAX, "too many heads in one call");
+    return launch("csa_merge_long_kernel", csa_merge_long_kernel<T>, dim3(static_cast<uint32_t>(bh * cbs)), dim3(256),
+                  0, stream, static_cast<const float*>(part_ml), static_cast<const float*>(part_acc),
+                  static_cast<T*>(out), static_cast<int>(D), static_cast<int>(tiles), static_cast<int>(cbs));
   });
 }
 
