@@ -451,28 +451,43 @@ __global__ __launch_bounds__(64) void csa_score_generic_kernel(const T* __restri
 }
 
 // Top-k per (b,h): keys -> LDS in one batch of loads (when they fit), then the
-// wavefront top-k of csa_device.hpp (register path of M keys per lane, or the
-// radix select).
+// wavefront top-k of csa_device.hpp (register path of M keys per lane), or for
+// more keys (M = 0) the workgroup's (k <= 64), else the radix select.
+constexpr int kTopkWaves = 4;  // wavefronts of the M = 0 kernel
+constexpr int kTopkListWords = kTopkWaves * (kWave + 1);
+
 template <int M, bool kInLds>
-__global__ __launch_bounds__(64) void csa_topk_kernel(const uint32_t* __restrict__ keys,
-                                                      int32_t* __restrict__ out, int64_t C, int k) {
-  extern __shared__ uint64_t lds64[];
+__global__ __launch_bounds__(M ? kWave : kTopkWaves * kWave) void csa_topk_kernel(const uint32_t* __restrict__ keys,
+                                                                                 int32_t* __restrict__ out, int64_t C,
+                                                                                 int k) {
+  extern __shared__ __align__(16) uint64_t lds64[];
   uint32_t* scratch = reinterpret_cast<uint32_t*>(lds64);
   uint32_t* hist = scratch + kTopkScratchWords;
   uint32_t* skey = hist + 256;
   int32_t* sidx = reinterpret_cast<int32_t*>(skey + k);
   uint32_t* counter = reinterpret_cast<uint32_t*>(sidx + k);
-  uint32_t* kl = counter + 1;
+  uint32_t* lists = counter + 1;  // block_topk's, M = 0 only
+  uint32_t* kl = lists + (M ? 0 : kTopkListWords);
   const int64_t bh = blockIdx.x;
   const uint32_t* kg = keys + bh * C;
   int32_t* o = out + bh * k;
   auto emit = [&](int r, int32_t i) { o[r] = i; };
-  if constexpr (kInLds) {
+  if constexpr (M > 0) {
     for (int i = threadIdx.x; i < C; i += kWave) kl[i] = kg[i];
     wave_lds_sync();
     wave_topk<M>(kl, static_cast<int>(C), k, scratch, hist, skey, sidx, counter, emit);
   } else {
-    wave_topk<M>(kg, static_cast<int>(C), k, scratch, hist, skey, sidx, counter, emit);
+    const uint32_t* src = kg;
+    if constexpr (kInLds) {
+      for (int i = threadIdx.x; i < C; i += kTopkWaves * kWave) kl[i] = kg[i];
+      src = kl;
+      __syncthreads();
+    }
+    if (k <= kWave &&
+        block_topk<kTopkWaves>(src, static_cast<int>(C), k, reinterpret_cast<unsigned long long*>(scratch), lists, emit))
+      return;
+    __syncthreads();
+    if (threadIdx.x < kWave) wave_topk<0>(src, static_cast<int>(C), k, scratch, hist, skey, sidx, counter, emit);
   }
 }
 
@@ -648,17 +663,23 @@ int csa_select_launch(const void* q, const float* summary, int32_t* out_indices,
                   static_cast<int>(D), scale);
   });
   if (rc != CSAHCA_OK) return rc;
-  const size_t base = kCandBytes + (256 + 2 * static_cast<size_t>(k) + 1) * sizeof(uint32_t);
+  // One wavefront with two keys per lane up to where 64 candidates hold the
+  // answer (see topk_regs_for); the workgroup otherwise.  Measured, 8 heads,
+  // registers against block_topk, us a call with the scores: top-32 of 64,
+  // 128, 256, 512: 4.5 / 5.1, 5.0 / 5.4, 5.7 / 5.3, 6.8 / 6.0; top-8 of 1024, 2048: 9.6
+  // / 6.6, 14.4 / 8.3; top-40, 48 of 128: 5.2 / 5.4, 11.7 / 5.3.
+  const int regs = k <= kWave && (C <= kWave || (C <= 2 * kWave && k <= 40)) ? 2 : 0;
+  const size_t base =
+      kCandBytes + (256 + 2 * static_cast<size_t>(k) + 1 + (regs ? 0 : kTopkListWords)) * sizeof(uint32_t);
   const bool in_lds = base + static_cast<size_t>(C) * sizeof(uint32_t) <= kLdsBudget;
   const size_t lds = base + (in_lds ? static_cast<size_t>(C) * sizeof(uint32_t) : 0);
   const dim3 grid(static_cast<uint32_t>(bh));
   const uint32_t* kp = keys;
   const int ki = static_cast<int>(k);
-  switch (topk_regs_for(C, k) * 2 + (in_lds ? 1 : 0)) {
-    case 17: return launch("csa_topk_kernel", csa_topk_kernel<8, true>, grid, dim3(kWave), lds, stream, kp, out_indices, C, ki);
-    case 65: return launch("csa_topk_kernel", csa_topk_kernel<32, true>, grid, dim3(kWave), lds, stream, kp, out_indices, C, ki);
-    case 1: return launch("csa_topk_kernel", csa_topk_kernel<0, true>, grid, dim3(kWave), lds, stream, kp, out_indices, C, ki);
-    default: return launch("csa_topk_kernel", csa_topk_kernel<0, false>, grid, dim3(kWave), lds, stream, kp, out_indices, C, ki);
+  switch (regs * 2 + (in_lds ? 1 : 0)) {
+    case 5: return launch("csa_topk_kernel", csa_topk_kernel<2, true>, grid, dim3(kWave), lds, stream, kp, out_indices, C, ki);
+    case 1: return launch("csa_topk_kernel", csa_topk_kernel<0, true>, grid, dim3(kTopkWaves * kWave), lds, stream, kp, out_indices, C, ki);
+    default: return launch("csa_topk_kernel", csa_topk_kernel<0, false>, grid, dim3(kTopkWaves * kWave), lds, stream, kp, out_indices, C, ki);
   }
 }
 

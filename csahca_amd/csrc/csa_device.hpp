@@ -289,6 +289,104 @@ __device__ bool wave_topk_regs(const uint32_t* keys, int C, int k, uint32_t* scr
   return true;
 }
 
+// ---------------------------------------------------------------------------
+// Top-k for k <= 64 over any number of keys, executed by all W wavefronts of a
+// workgroup (W 4 or 8): the steps of wave_topk_regs with the keys read again
+// from memory instead of held in registers, so no wavefront scans more than
+// C / W of them.
+//   1. each lane takes the maximum of its C / (64 W) keys (row j of 64 W
+//      positions rotated by j, as there), each wavefront sorts its 64 maxima;
+//   2. every wavefront merges the W sorted lists to the 64 largest maxima (the
+//      larger of a lane and its mirror in the next list, then one bitonic
+//      merge) and takes the k-th: t;
+//   3. keys >= t are compacted into LDS composites: lane counts, a prefix
+//      inside the wavefront by ballots per bit of the count, the wavefronts'
+//      totals through LDS;
+//   4. thread j ranks composite j.
+// Returns false in every thread (nothing emitted) when more than kBlockCand
+// keys are >= t (about 64 W ln(64 W / (64 W - k)) are, of independent keys: 74
+// for k = 64 at W = 4) or when t == 0.  cand: kBlockCand composites, 16-byte
+// aligned; lists: W * 65 words.  Contains barriers; the caller orders the last
+// reads of cand and lists.
+// Bound by its chain of LDS round trips and, from a few thousand keys, by the
+// reads: C / (64 W) a lane, twice.  (One wavefront's radix select, the only
+// path above 2048 keys before, reads every key 6 times with LDS atomics: B1 H8
+// D128 f32, 6295 chunks, top-14: 66.1 us a step, with this 23.2; B2 H8 D64 f32,
+// 3142 chunks, top-56: 43.8, 16.6.)
+// ---------------------------------------------------------------------------
+constexpr int kBlockCand = 192;
+
+template <int W, typename Out>
+__device__ bool block_topk(const uint32_t* keys, int C, int k, unsigned long long* cand, uint32_t* lists, Out out) {
+  constexpr int NT = W * kWave;
+  const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
+  const int rows = (C + NT - 1) / NT;
+  auto pos_of = [&](int j) { return NT * j + ((tid - j) & (NT - 1)); };
+  uint32_t mx = 0;
+#pragma unroll 4
+  for (int j = 0; j < rows; ++j) {
+    const int i = pos_of(j);
+    const uint32_t v = keys[i < C ? i : C - 1];  // (the last key again: a key of the set, at no lane of its own)
+    mx = (i < C && v > mx) ? v : mx;
+  }
+  lists[wave * kWave + lane] = wave_sort_desc(mx, lane);
+  for (int i = tid; i < kBlockCand; i += NT) cand[i] = 0ull;  // below every composite
+  __syncthreads();
+  uint32_t top = lists[lane];
+#pragma unroll
+  for (int w = 1; w < W; ++w) {
+    const uint32_t o = lists[w * kWave + (kWave - 1 - lane)];
+    top = merge_desc<32>(top > o ? top : o, lane);
+  }
+  const uint32_t t = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(top), k - 1));
+  if (t == 0u) return false;
+  int cnt = 0;
+#pragma unroll 4
+  for (int j = 0; j < rows; ++j) {
+    const int i = pos_of(j);
+    const uint32_t v = keys[i < C ? i : C - 1];
+    cnt += (i < C && v >= t) ? 1 : 0;
+  }
+  int slot = 0, n = 0;
+  for (int b = 0; (1 << b) <= rows; ++b) {
+    const unsigned long long bal = __ballot((cnt >> b) & 1);
+    slot += lanes_below(bal) << b;
+    n += __popcll(bal) << b;
+  }
+  if (lane == 0) lists[W * kWave + wave] = static_cast<uint32_t>(n);
+  __syncthreads();
+  int total = 0;
+#pragma unroll
+  for (int w = 0; w < W; ++w) {
+    const int nw = static_cast<int>(lists[W * kWave + w]);
+    slot += w < wave ? nw : 0;
+    total += nw;
+  }
+  if (total > kBlockCand) return false;
+  if (cnt > 0) {
+    for (int j = 0; j < rows; ++j) {
+      const int i = pos_of(j);
+      const uint32_t v = keys[i < C ? i : C - 1];
+      if (i < C && v >= t)
+        cand[slot++] = (static_cast<unsigned long long>(v) << 32) | static_cast<uint32_t>(~static_cast<uint32_t>(i));
+    }
+  }
+  __syncthreads();
+  if (tid < total) {
+    const unsigned long long cj = cand[tid];
+    int r = 0;
+    for (int b = 0; b < total; b += 16) {  // (kBlockCand is a multiple of 16; slots past the total hold 0)
+      ulonglong2 c2[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) c2[i] = *reinterpret_cast<const ulonglong2*>(cand + b + 2 * i);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) r += (c2[i].x > cj) + (c2[i].y > cj);
+    }
+    if (r < k) out(r, static_cast<int32_t>(~static_cast<uint32_t>(cj)));
+  }
+  return true;
+}
+
 // Position of the largest key of keys[0, C) (1 <= C <= 64 * M), larger key
 // first and equal keys by lower position: the first slot of every top-k
 // above.  Each lane reads its M keys in one batch (position 64 j + lane;
@@ -330,10 +428,19 @@ __device__ __forceinline__ int32_t wave_top1(const uint32_t* keys, int C) {
   return static_cast<int32_t>(~static_cast<uint32_t>(c));
 }
 
-// Register-path size for a selection: keys per lane M (C <= 64 * M), or 0 for
-// the LDS radix path only.  Kernels take M as a template parameter so each
-// instantiation carries exactly one register path.
+// Register-path size for the fused step's selection: keys per lane M (C <= 64
+// * M), or 0 for block_topk (k <= 64) or the radix select.  Kernels take M as a
+// template parameter so each instantiation carries exactly one of them.  The
+// register path fails where more than 64 keys reach its threshold, which of
+// independent keys 64 ln(64 / (64 - k)) do (44 for k = 32, 63 for 40, 89 for
+// 48), fewer of at most 2 per lane; the radix select behind it costs 6-24 us.
+// Measured, B1 H8 D128 chunk 16, registers against block_topk, us a step:
+// top-32 of 512, 1024, 2048: 8.5 / 9.4, 10.95 / 11.1, 12.5 / 13.0; top-40 of 64,
+// 128, 256: 9.3 / 10.0, 9.3 / 9.8, 16.1 / 9.8; top-64 of 64, 128, 512, 2048: 9.6 /
+// 10.2, 18.3 / 10.7, 21.4 / 11.5, 36.2 / 13.7.
 inline int topk_regs_for(int64_t C, int64_t k) {
+  if (C > 64 && k > 40) return 0;
+  if (C > 128 && k > 32) return 0;
   if (k > kWave) return 0;
   if (C <= 512) return 8;
   if (C <= 2048) return 32;

@@ -453,7 +453,7 @@ __device__ __forceinline__ void csa_step_body(StepParams a, uint32_t block) {
                             tok_first);
     }
   }
-  if (wave == 0) {
+  {
     int32_t* io = a.idx_out + h * a.topk;
     const bool write_ids = (p == 0);
     auto emit = [&](int r, int32_t i) {
@@ -463,8 +463,21 @@ __device__ __forceinline__ void csa_step_body(StepParams a, uint32_t block) {
     // Fewer chunks in play than selection slots (device count only): the
     // slots past the count hold -1, which the attention below skips.
     const int kk = static_cast<int>(min<int64_t>(a.topk, C));
-    if (kk > 0) wave_topk<TOPK_M>(keys_l, static_cast<int>(C), kk, tk_scratch, hist, skey, sidx, lcount, emit);
-    for (int r = kk + lane; r < a.topk; r += kWave) emit(r, -1);
+    // More keys than the register top-k holds: all wavefronts select together
+    // (candidates over the wavefront top-k's scratch and the histogram, lists
+    // over the state exchange of phase C).
+    bool done = kk <= 0;
+    if constexpr (TOPK_M == 0) {
+      static_assert(2 * kBlockCand <= kTopkScratchWords + 256, "candidates fit the top-k scratch and the histogram");
+      static_assert(W * (kWave + 1) <= W * (D + 2), "lists fit the state exchange");
+      if (kk > 0 && kk <= kWave)
+        done = block_topk<W>(keys_l, static_cast<int>(C), kk, reinterpret_cast<unsigned long long*>(tk_scratch),
+                             reinterpret_cast<uint32_t*>(comb), emit);
+    }
+    if (wave == 0) {
+      if (!done) wave_topk<TOPK_M>(keys_l, static_cast<int>(C), kk, tk_scratch, hist, skey, sidx, lcount, emit);
+      for (int r = max(kk, 0) + lane; r < a.topk; r += kWave) emit(r, -1);
+    }
   }
   __syncthreads();
   CSAHCA_STAMP(3);
