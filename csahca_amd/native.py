@@ -895,17 +895,19 @@ def dsv4_decode_forward_tiled(q, paged_k_cache_u8, token_indices, topk_lengths, 
     if not (q.is_cuda and paged_k_cache_u8.is_cuda and token_indices.is_cuda):
         raise RuntimeError("q, paged_k_cache_u8, and token_indices must be CUDA tensors")
     _dsv4_common(q, paged_k_cache_u8, token_indices, topk_lengths, attn_sink, page_size, allow_empty=True)
-    if paged_k_cache_u8.shape[1] % 4 != 0:
+    num_pages, bpp = paged_k_cache_u8.shape
+    if bpp % 4 != 0:
         raise RuntimeError("tiled DSV4 kernel requires bytes_per_page divisible by 4 for vectorized loads")
-    nq, heads = q.shape[0], q.shape[1]
+    nq, heads, _ = q.shape
+    slots = token_indices.shape[1]
     has_extra = (extra_paged_k_cache_u8 is not None and extra_paged_k_cache_u8.numel() > 0
                  and extra_token_indices is not None and extra_token_indices.numel() > 0)
-    extra_slots = 0
+    extra_slots = extra_pages = ebpp = 0
     if has_extra:
         _dsv4_extra_checks(extra_paged_k_cache_u8, extra_token_indices, extra_topk_lengths, nq, q.get_device())
         if extra_page_size <= 0:
             raise RuntimeError("extra_page_size must be positive")
-        ebpp = extra_paged_k_cache_u8.shape[1]
+        extra_pages, ebpp = extra_paged_k_cache_u8.shape
         if ebpp < extra_page_size * (576 + 8):
             raise RuntimeError("extra_bytes_per_page is too small for DSV4 page layout")
         if ebpp % 4 != 0:
@@ -921,17 +923,19 @@ def dsv4_decode_forward_tiled(q, paged_k_cache_u8, token_indices, topk_lengths, 
     if nq == 0 or heads == 0:
         return out
     stream = _raw_stream(dev)
-    ws = _scratch_workspace(_ws_bytes("csahca_dsv4_decode_workspace_bytes", nq, heads, token_indices.shape[1],
-                                      extra_slots, tile_size), dev, stream)
-    ec = extra_paged_k_cache_u8 if has_extra else None
-    _rc(lib().csahca_dsv4_decode_forward_tiled(
-        q.data_ptr(), _DTYPES[q.dtype], nq, heads, paged_k_cache_u8.data_ptr(), paged_k_cache_u8.shape[0],
-        paged_k_cache_u8.shape[1], page_size, token_indices.data_ptr(), token_indices.shape[1],
-        _ptr(_opt(topk_lengths)), _ptr(ec), ec.shape[0] if has_extra else 0,
-        ec.shape[1] if has_extra else 0, extra_page_size if has_extra else 1,
-        _ptr(extra_token_indices) if has_extra else None, extra_slots,
-        _ptr(_opt(extra_topk_lengths)) if has_extra else None, _ptr(_opt(attn_sink)), float(softmax_scale),
-        tile_size, out.data_ptr(), ws.data_ptr(), ws.numel(), stream))
+    ws = _scratch_workspace(_ws_bytes("csahca_dsv4_decode_workspace_bytes", nq, heads, slots, extra_slots, tile_size),
+                            dev, stream)
+    rc = lib().csahca_dsv4_decode_forward_tiled(
+        q.data_ptr(), _DTYPES[q.dtype], nq, heads, paged_k_cache_u8.data_ptr(), num_pages, bpp, page_size,
+        token_indices.data_ptr(), slots,
+        None if topk_lengths is None or topk_lengths.numel() == 0 else topk_lengths.data_ptr(),
+        extra_paged_k_cache_u8.data_ptr() if has_extra else None, extra_pages, ebpp,
+        extra_page_size if has_extra else 1, extra_token_indices.data_ptr() if has_extra else None, extra_slots,
+        _ptr(_opt(extra_topk_lengths)) if has_extra else None,
+        None if attn_sink is None or attn_sink.numel() == 0 else attn_sink.data_ptr(), float(softmax_scale),
+        tile_size, out.data_ptr(), ws.data_ptr(), ws.numel(), stream)
+    if rc != 0:
+        _rc(rc)
     return out
 
 
