@@ -15,17 +15,22 @@
 //                     means, scores the K mean against q and writes the
 //                     score (scores[b,h,c]) and the V mean (means[b,h,c,:])
 //                     to the workspace;
+//   hybrid_chunk_kernel  the chunk pass above and the CSA summaries of the same
+//                     K rows, from one read of K (the hybrid op that builds its
+//                     own summaries): one wavefront per chunk and tensor;
 //   hca_merge_kernel  one workgroup per (b, h, block of 32 output columns):
 //                     softmax over the C scores, probabilities rounded to the
 //                     storage type, sum of its columns of the V means,
 //                     optional blend with a CSA output.  Spreading a head's
 //                     columns over workgroups keeps each one to a single round
 //                     trip of ~C x 128 bytes even at batch 1.
+#include "csa_device.hpp"
 #include "hca_device.hpp"
 
 #include <algorithm>
 #include <climits>
 #include <cmath>
+#include <cstdlib>
 
 namespace csahca {
 namespace {
@@ -44,6 +49,118 @@ __global__ __launch_bounds__(kHcaThreads) void hca_chunk_kernel(const T* __restr
                                                               float* __restrict__ scores,
                                                               float* __restrict__ means, float scale) {
   hca_chunk_body<T, kVec>(q, k, v, scores, means, S, D, chunk, C, scale, blockIdx.x);
+}
+
+// The HCA chunk pass and the CSA chunk summaries from one read of K and V.
+// Wavefront 2i of the grid takes K of HCA chunk i, wavefront 2i + 1 its V, in
+// the summary kernel's lane split: lane (grp, col) takes rows grp, grp + RPL,
+// ... of VEC columns.  Of the rows one lane adds, every fourth belongs to the
+// same row group of hca_chunk_body (256 / LPR = 4 RPL groups), so it keeps 4
+// group sums, in that body's order, beside the running sum of the CSA chunk:
+// both results have the bits of the separate kernels.  HBM-bound: kHybridRows
+// 16-byte loads in flight per lane, no barrier.  (Measured, B2 H8 S32768 D128
+// bf16, chunks 64 and 256, us a hybrid call: the summary kernel, then the step
+// beside the HCA pass, 71.2; this kernel, then the step, 64.4.  8 loads: level
+// where wavefronts fill the chip, 20% slower where they do not, 256 of them on
+// 128 MiB.)
+constexpr int kHybridRows = 16;
+constexpr int kHybridWaves = 4;
+
+template <typename T, int D>
+__global__ __launch_bounds__(kHybridWaves * kWave) void hybrid_chunk_kernel(
+    const T* __restrict__ k, const T* __restrict__ v, int64_t items, int hca_chunk, int csa_chunk,
+    float* __restrict__ summary, const T* __restrict__ q, uint32_t hca_chunks, float* __restrict__ scores,
+    float* __restrict__ means, float scale) {
+  using L = AttendLayout<T, D>;
+  constexpr int VEC = L::VEC, LPR = L::LPR, RPL = L::RPL;
+  constexpr int G = 4;                // group sums per lane
+  constexpr int R = G * RPL;          // row groups of hca_chunk_body
+  constexpr int U = kHybridRows;
+  static_assert(R * LPR == kHcaThreads && U % G == 0, "the row groups of hca_chunk_body");
+  __shared__ __align__(16) float sums[kHybridWaves][R * D];
+  const int lane = threadIdx.x % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int grp = lane / LPR, col = lane % LPR;
+  const int64_t item = static_cast<int64_t>(blockIdx.x) * (kHybridWaves / 2) + wave / 2;
+  if (item >= items) return;
+  const bool is_k = (wave & 1) == 0;
+  // S is a multiple of both chunk sizes: chunks lie end to end over all heads.
+  const T* __restrict__ base = (is_k ? k : v) + item * hca_chunk * D + col * VEC;
+  float* __restrict__ dst = summary + item * (hca_chunk / csa_chunk) * D + col * VEC;
+  const float fc = static_cast<float>(csa_chunk);
+  float hs[G][VEC], acc[VEC];
+#pragma unroll
+  for (int e = 0; e < VEC; ++e) {
+    acc[e] = 0.f;
+#pragma unroll
+    for (int g = 0; g < G; ++g) hs[g][e] = 0.f;
+  }
+  int left = csa_chunk;  // rows of the open CSA chunk not yet added
+  for (int r0 = 0; r0 < hca_chunk; r0 += U * RPL) {
+    uint4 x[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {  // (rows past the chunk read its last rows again)
+      const int r = r0 + (u / G) * R < hca_chunk ? r0 + u * RPL : hca_chunk - R + (u % G) * RPL;
+      x[u] = load_global_u4(base + static_cast<int64_t>(r + grp) * D);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int b = 0; b < U / G; ++b) {
+      if (r0 + b * R < hca_chunk) {
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+          float f[VEC];
+          widen16<T>(x[b * G + g], f);
+#pragma unroll
+          for (int e = 0; e < VEC; ++e) {
+            hs[g][e] += f[e];
+            acc[e] += f[e];
+          }
+        }
+        left -= R;
+        if (left == 0) {
+          left = csa_chunk;
+          if (is_k) {
+#pragma unroll
+            for (int off = LPR; off < kWave; off <<= 1)
+#pragma unroll
+              for (int e = 0; e < VEC; ++e) acc[e] += xor_lanes(acc[e], off);
+            if (grp == 0) {
+#pragma unroll
+              for (int e = 0; e < VEC; ++e) dst[e] = acc[e] / fc;
+            }
+            dst += D;
+          }
+#pragma unroll
+          for (int e = 0; e < VEC; ++e) acc[e] = 0.f;
+        }
+      }
+    }
+  }
+  float* s = sums[wave];
+#pragma unroll
+  for (int g = 0; g < G; ++g)
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) s[(grp + g * RPL) * D + col * VEC + e] = hs[g][e];
+  wave_lds_sync();
+  const float inv_n = 1.f / static_cast<float>(hca_chunk);
+  const T* qp = q + static_cast<int64_t>(static_cast<uint32_t>(item) / hca_chunks) * D;
+  float dot = 0.f;
+#pragma unroll
+  for (int d0 = 0; d0 < D; d0 += kWave) {
+    const int d = d0 + lane;
+    float a = 0.f;
+#pragma unroll
+    for (int g = 0; g < R; ++g) a += s[g * D + d];
+    const float m = round_to<T>(a * inv_n);
+    if (is_k) {
+      const float part = wave_sum(fmaf(to_f32(qp[d]), m, 0.f));
+      dot = d0 == 0 ? part : dot + part;
+    } else {
+      means[item * D + d] = m;
+    }
+  }
+  if (is_k && lane == 0) scores[item] = dot * scale;
 }
 
 // Merge thread layout: 32 columns x 8 row groups; a wavefront reads 2 rows of
@@ -157,6 +274,36 @@ namespace {
 size_t hca_means_offset(int64_t n_scores) {
   return (static_cast<size_t>(n_scores) * sizeof(float) + 255) & ~size_t{255};
 }
+
+// CSAHCA_HYBRID_ONE_READ=0 / 1 turns hybrid_chunk_kernel off / on wherever it
+// applies (read per call); unset (-1): the rule of hybrid_one_read.
+int env_one_read() {
+  const char* s = std::getenv("CSAHCA_HYBRID_ONE_READ");
+  return s ? (std::atoi(s) != 0 ? 1 : 0) : -1;
+}
+
+// Whether the hybrid op that builds its own summaries reads K once
+// (hybrid_chunk_kernel).  A wavefront walks a whole HCA chunk, so one of more
+// than 128 KiB needs many beside it.  With head_dim 128 in 16 bits the other
+// route runs the step beside the HCA pass, which hides it: there the second
+// read of K has to cost more than the step, from about 48 MiB of K.  Measured,
+// us a call, one read / two:
+//   bf16 D128: B8 H8 S16384 115 / 146, B1 H8 S32768 34.9 / 37.5, B1 H8 S16384
+//   24.9 / 24.5, S8192 21.7 / 18.5; HCA chunks of 2048: 70.6 / 72.3;
+//   D64 f16 B4 H8 S16384 35.0 / 46.2, B1 H4 S2048 16.4 / 17.4; f32 D128 B1 H8
+//   S16384 34.4 / 44.6, S2048 23.1 / 24.2; f32 D256 B1 H4 S4096 with 64
+//   wavefronts of 512 KiB 53.3 / 52.2.
+bool hybrid_one_read(int dtype, int64_t head_dim, int64_t csa_chunk, int64_t hca_chunk, int64_t items) {
+  if (dtype == CSAHCA_F64 || (head_dim != 64 && head_dim != 128 && head_dim != 256)) return false;
+  const int64_t esz = dtype == CSAHCA_F32 ? 4 : 2;
+  if (hca_chunk % csa_chunk != 0 || csa_chunk % (kHcaThreads * (16 / esz) / head_dim) != 0)
+    return false;  // whole CSA chunks of whole row groups
+  const int env = env_one_read();
+  if (env >= 0) return env == 1;
+  const int64_t bytes = hca_chunk * head_dim * esz;
+  if (bytes > 128 * 1024 && items < 512) return false;
+  return esz == 4 || head_dim != 128 || items * bytes >= (int64_t{48} << 20);
+}
 }  // namespace
 
 extern "C" size_t csahca_hca_decode_workspace_bytes(int64_t batch, int64_t heads, int64_t seq_len,
@@ -242,3 +389,59 @@ int hca_merge_launch(int dtype, void* workspace, const void* blend_src, double b
 size_t hca_workspace_means_offset(int64_t n_scores) { return hca_means_offset(n_scores); }
 
 }  // namespace csahca
+
+extern "C" int csahca_hybrid_decode_forward_build(const void* q, const void* k_cache, const void* v_cache,
+                                                  float* summary, void* csa_out, int32_t* csa_indices, void* out,
+                                                  int dtype, int64_t batch, int64_t heads, int64_t seq_len,
+                                                  int64_t head_dim, int64_t csa_chunk_size, int64_t top_k,
+                                                  int64_t hca_chunk_size, double csa_weight, void* step_workspace,
+                                                  size_t step_workspace_bytes, void* hca_workspace,
+                                                  size_t hca_workspace_bytes, void* stream_ptr) {
+  clear_error();
+  CSAHCA_REQUIRE(valid_dtype(dtype), "q, k_cache and v_cache must be float32, float64, float16 or bfloat16");
+  CSAHCA_REQUIRE(batch >= 0 && heads >= 0 && seq_len >= 0 && head_dim >= 0, "negative dimension");
+  CSAHCA_REQUIRE(csa_chunk_size > 0 && csa_chunk_size <= INT_MAX, "chunk_size must be positive");
+  CSAHCA_REQUIRE(hca_chunk_size > 0 && hca_chunk_size <= INT_MAX, "chunk_size must be positive");
+  CSAHCA_REQUIRE(seq_len % csa_chunk_size == 0 && seq_len % hca_chunk_size == 0,
+                 "seq length must be divisible by chunk_size");
+  const int64_t bh = batch * heads, C = seq_len / csa_chunk_size, Ch = seq_len / hca_chunk_size;
+  const size_t need = csahca_hca_decode_workspace_bytes(batch, heads, seq_len, head_dim, hca_chunk_size);
+  const bool one_read = bh > 0 && Ch > 0 && bh * Ch <= INT32_MAX && q && k_cache && v_cache && out && csa_out && summary &&
+                  hca_workspace != nullptr && hca_workspace_bytes >= need &&
+                  ((reinterpret_cast<uintptr_t>(k_cache) | reinterpret_cast<uintptr_t>(v_cache)) % 16) == 0 &&
+                  hybrid_one_read(dtype, head_dim, csa_chunk_size, hca_chunk_size, bh * Ch);
+  if (!one_read) {
+    const int rc = csahca_csa_chunk_summary(k_cache, summary, dtype, batch, heads, seq_len, head_dim, csa_chunk_size,
+                                            C, 0, C, stream_ptr);
+    if (rc != CSAHCA_OK) return rc;
+    return csahca_hybrid_decode_forward(q, k_cache, v_cache, summary, csa_out, csa_indices, out, dtype, batch, heads,
+                                        seq_len, head_dim, C, csa_chunk_size, top_k, hca_chunk_size, csa_weight,
+                                        step_workspace, step_workspace_bytes, hca_workspace, hca_workspace_bytes,
+                                        stream_ptr);
+  }
+  hipStream_t stream = static_cast<hipStream_t>(stream_ptr);
+  float* scores = static_cast<float*>(hca_workspace);
+  float* means = reinterpret_cast<float*>(static_cast<char*>(hca_workspace) + hca_means_offset(bh * Ch));
+  const float scale = static_cast<float>(1.0 / std::sqrt(static_cast<double>(head_dim)));
+  auto run = [&](auto tag, auto dim) -> int {
+    using T = decltype(tag);
+    constexpr int D = decltype(dim)::value;
+    return launch("hybrid_chunk_kernel", hybrid_chunk_kernel<T, D>,
+                  dim3(static_cast<uint32_t>(ceil_div(bh * Ch, int64_t{kHybridWaves / 2}))),
+                  dim3(kHybridWaves * kWave), 0, stream, static_cast<const T*>(k_cache),
+                  static_cast<const T*>(v_cache), bh * Ch, static_cast<int>(hca_chunk_size),
+                  static_cast<int>(csa_chunk_size), summary, static_cast<const T*>(q), static_cast<uint32_t>(Ch),
+                  scores, means, scale);
+  };
+  auto with_dim = [&](auto tag) -> int {
+    if (head_dim == 64) return run(tag, std::integral_constant<int, 64>{});
+    if (head_dim == 128) return run(tag, std::integral_constant<int, 128>{});
+    return run(tag, std::integral_constant<int, 256>{});
+  };
+  int rc = dtype == CSAHCA_BF16 ? with_dim(bf16{}) : dtype == CSAHCA_F16 ? with_dim(f16{}) : with_dim(0.0f);
+  if (rc != CSAHCA_OK) return rc;
+  rc = csahca_csa_decode_step(q, k_cache, v_cache, summary, csa_out, csa_indices, dtype, batch, heads, seq_len,
+                              head_dim, C, csa_chunk_size, top_k, step_workspace, step_workspace_bytes, stream_ptr);
+  if (rc != CSAHCA_OK) return rc;
+  return hca_merge_launch(dtype, hca_workspace, csa_out, csa_weight, out, bh, Ch, static_cast<int>(head_dim), stream);
+}

@@ -75,6 +75,8 @@ _SIGNATURES = {
     "csahca_hca_decode_forward": (_int, [_vp, _vp, _vp, _vp, _dbl, _vp, _int] + [_i64] * 5 + [_vp, _sz, _vp]),
     "csahca_hybrid_decode_forward": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _int] + [_i64] * 8 + [_dbl] +
                                      [_vp, _sz, _vp, _sz, _vp]),
+    "csahca_hybrid_decode_forward_build": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _int] + [_i64] * 7 + [_dbl] +
+                                           [_vp, _sz, _vp, _sz, _vp]),
     "csahca_block_linear": (_int, [_vp, _vp, _dbl, _vp, _int, _vp, _vp, _dbl, _vp, _int, _i64, _i64, _i64, _vp,
                                    _vp]),
     "csahca_block_qkv": (_int, [_vp, _vp, _dbl, _vp, _vp, _vp, _vp, _vp, _vp, _int] + [_i64] * 5 + [_vp]),
@@ -746,11 +748,16 @@ def hybrid_decode_forward(q, k_cache, v_cache, *, csa_chunk_size: int, csa_top_k
     CSA decode step (selection from the chunk summaries of K, built here when
     ``summary`` is None) blended with HCA at ``csa_weight``.  Building the
     summary here needs whole chunks, as chunk_mean does (reference.py:40-42)."""
-    if summary is None:
+    build = summary is None
+    if build:
         _check(int(csa_chunk_size) > 0, "chunk_size must be positive")
         _check(k_cache.dim() == 4 and k_cache.shape[2] % int(csa_chunk_size) == 0,
                "seq length must be divisible by chunk_size")
-        summary = csa_chunk_summary(k_cache, csa_chunk_size)
+        _check(k_cache.is_cuda, "k_cache must be CUDA")
+        _check(k_cache.is_contiguous(), "k_cache must be contiguous")
+        _check(k_cache.dtype in _FLOATING, f"unsupported dtype {k_cache.dtype}")
+        summary = torch.empty((*k_cache.shape[:2], k_cache.shape[2] // int(csa_chunk_size), k_cache.shape[3]),
+                              dtype=torch.float32, device=k_cache.device)
     csa_chunk_size, csa_top_k, hca_chunk_size = int(csa_chunk_size), int(csa_top_k), int(hca_chunk_size)
     _csa_checks(q, k_cache, v_cache, None, csa_chunk_size, tiled=False)
     _check(summary.is_cuda and summary.is_contiguous() and summary.dtype == torch.float32 and summary.dim() == 4,
@@ -769,10 +776,14 @@ def hybrid_decode_forward(q, k_cache, v_cache, *, csa_chunk_size: int, csa_top_k
         sws = _step_workspace(lib().csahca_csa_step_workspace_bytes(B, H, C, D, csa_top_k, csa_chunk_size), q.device,
                               (B * H, C, D, k, csa_chunk_size))
         hws = _workspace(lib().csahca_hca_decode_workspace_bytes(B, H, S, D, hca_chunk_size), q.device)
-        _rc(lib().csahca_hybrid_decode_forward(_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(summary), _ptr(csa_out),
-                                               _ptr(idx), _ptr(out), _DTYPES[q.dtype], B, H, S, D, C, csa_chunk_size,
-                                               csa_top_k, hca_chunk_size, float(csa_weight), _ptr(sws), sws.numel(),
-                                               _ptr(hws), hws.numel(), _stream()))
+        head = (_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(summary), _ptr(csa_out), _ptr(idx), _ptr(out),
+                _DTYPES[q.dtype], B, H, S, D)
+        tail = (csa_chunk_size, csa_top_k, hca_chunk_size, float(csa_weight), _ptr(sws), sws.numel(), _ptr(hws),
+                hws.numel(), _stream())
+        if build:
+            _rc(lib().csahca_hybrid_decode_forward_build(*head, *tail))
+        else:
+            _rc(lib().csahca_hybrid_decode_forward(*head, C, *tail))
     return out
 
 

@@ -262,6 +262,20 @@ int csahca_hybrid_decode_forward(const void* q, const void* k_cache, const void*
                                  void* step_workspace, size_t step_workspace_bytes, void* hca_workspace,
                                  size_t hca_workspace_bytes, void* stream);
 
+/* csahca_hybrid_decode_forward with the summaries built by the call:
+ * summary [B, H, seq_len/csa_chunk_size, D] fp32 is an output, with the bits of
+ * csahca_csa_chunk_summary, and seq_len must be a multiple of both chunk sizes.
+ * Where hca_chunk_size is a multiple of csa_chunk_size and the shape allows it
+ * (head_dim 64, 128 or 256, not float64, 16-byte aligned tensors) one kernel
+ * reads K and V once for the summaries and the HCA chunk pass; elsewhere the two
+ * calls run in turn. */
+int csahca_hybrid_decode_forward_build(const void* q, const void* k_cache, const void* v_cache, float* summary,
+                                       void* csa_out, int32_t* csa_indices, void* out, int dtype, int64_t batch,
+                                       int64_t heads, int64_t seq_len, int64_t head_dim, int64_t csa_chunk_size,
+                                       int64_t top_k, int64_t hca_chunk_size, double csa_weight,
+                                       void* step_workspace, size_t step_workspace_bytes, void* hca_workspace,
+                                       size_t hca_workspace_bytes, void* stream);
+
 /* ------------------------------------------------------------------------- */
 /* DSV4: MQA decode over the paged FP8 latent cache                           */
 /* ------------------------------------------------------------------------- */
