@@ -828,6 +828,14 @@ StepKernelFn step_kernel_merge(int64_t head_dim, int m, bool pos) {
   if (m == 8)                                                                                          \
     return pos ? csa_step_kernel<T, DD, 8, true, false, kStepWaves, MG>                               \
                : csa_step_kernel<T, DD, 8, false, false, kStepWaves, MG>;                             \
+  if constexpr (DD == 128 && sizeof(T) == 2) {                                                         \
+    if (m == 2)                                                                                        \
+      return pos ? csa_step_kernel<T, DD, 2, true, false, kStepWaves, MG>                              \
+                 : csa_step_kernel<T, DD, 2, false, false, kStepWaves, MG>;                            \
+    if (m == 16)                                                                                       \
+      return pos ? csa_step_kernel<T, DD, 16, true, false, kStepWaves, MG>                             \
+                 : csa_step_kernel<T, DD, 16, false, false, kStepWaves, MG>;                           \
+  }                                                                                                    \
   if (m == 32)                                                                                         \
     return pos ? csa_step_kernel<T, DD, 32, true, false, kStepWaves, MG>                              \
                : csa_step_kernel<T, DD, 32, false, false, kStepWaves, MG>;                            \
@@ -857,14 +865,21 @@ StepKernelFn step_kernel_for_dtype(int dtype, int64_t head_dim, int m, bool pos,
 // per CU (no neighbour to overlap a workgroup's memory waits with; measured:
 // B32 top-8 4-8% faster, and ~1% slower where two workgroups share a CU).
 // bf16/f16, head_dim 128, count modes; nullptr elsewhere.
+template <typename T>
+StepKernelFn step_kernel_pipelined_for(int m) {
+  switch (m) {
+    case 2: return csa_step_kernel<T, 128, 2, false, true>;
+    case 8: return csa_step_kernel<T, 128, 8, false, true>;
+    case 16: return csa_step_kernel<T, 128, 16, false, true>;
+    case 32: return csa_step_kernel<T, 128, 32, false, true>;
+    default: return csa_step_kernel<T, 128, 0, false, true>;
+  }
+}
+
 StepKernelFn step_kernel_pipelined(int dtype, int64_t head_dim, int m) {
   if (head_dim != 128) return nullptr;
-  if (dtype == CSAHCA_BF16)
-    return m == 8 ? csa_step_kernel<bf16, 128, 8, false, true>
-                  : m == 32 ? csa_step_kernel<bf16, 128, 32, false, true> : csa_step_kernel<bf16, 128, 0, false, true>;
-  if (dtype == CSAHCA_F16)
-    return m == 8 ? csa_step_kernel<f16, 128, 8, false, true>
-                  : m == 32 ? csa_step_kernel<f16, 128, 32, false, true> : csa_step_kernel<f16, 128, 0, false, true>;
+  if (dtype == CSAHCA_BF16) return step_kernel_pipelined_for<bf16>(m);
+  if (dtype == CSAHCA_F16) return step_kernel_pipelined_for<f16>(m);
   return nullptr;
 }
 
@@ -875,16 +890,21 @@ StepKernelFn step_kernel_pipelined(int dtype, int64_t head_dim, int m) {
 // elsewhere.  (8 wavefronts: at 256 heads with top-32 selections 1-4% faster
 // than 16, whose extra loads in flight one CU cannot return any faster.)
 constexpr int kWideWaves = 8;
+template <typename T>
+StepKernelFn step_kernel_wide_for(int m) {
+  switch (m) {
+    case 2: return csa_step_kernel<T, 128, 2, false, true, kWideWaves, kMergeRegs>;
+    case 8: return csa_step_kernel<T, 128, 8, false, true, kWideWaves, kMergeRegs>;
+    case 16: return csa_step_kernel<T, 128, 16, false, true, kWideWaves, kMergeRegs>;
+    case 32: return csa_step_kernel<T, 128, 32, false, true, kWideWaves, kMergeRegs>;
+    default: return csa_step_kernel<T, 128, 0, false, true, kWideWaves, kMergeRegs>;
+  }
+}
+
 StepKernelFn step_kernel_wide(int dtype, int64_t head_dim, int m) {
   if (head_dim != 128) return nullptr;
-  if (dtype == CSAHCA_BF16)
-    return m == 8    ? csa_step_kernel<bf16, 128, 8, false, true, kWideWaves, kMergeRegs>
-           : m == 32 ? csa_step_kernel<bf16, 128, 32, false, true, kWideWaves, kMergeRegs>
-                     : csa_step_kernel<bf16, 128, 0, false, true, kWideWaves, kMergeRegs>;
-  if (dtype == CSAHCA_F16)
-    return m == 8    ? csa_step_kernel<f16, 128, 8, false, true, kWideWaves, kMergeRegs>
-           : m == 32 ? csa_step_kernel<f16, 128, 32, false, true, kWideWaves, kMergeRegs>
-                     : csa_step_kernel<f16, 128, 0, false, true, kWideWaves, kMergeRegs>;
+  if (dtype == CSAHCA_BF16) return step_kernel_wide_for<bf16>(m);
+  if (dtype == CSAHCA_F16) return step_kernel_wide_for<f16>(m);
   return nullptr;
 }
 
@@ -915,12 +935,19 @@ uint32_t env_step_test_timeout() {
   return n > 0 ? static_cast<uint32_t>(std::min<long long>(n, kSpinLimit)) : 0;
 }
 
+template <typename T>
+HybridKernelFn hybrid_kernel_pick(int m) {
+  switch (m) {
+    case 2: return csa_hybrid_kernel<T, 128, 2>;
+    case 8: return csa_hybrid_kernel<T, 128, 8>;
+    case 16: return csa_hybrid_kernel<T, 128, 16>;
+    case 32: return csa_hybrid_kernel<T, 128, 32>;
+    default: return csa_hybrid_kernel<T, 128, 0>;
+  }
+}
+
 HybridKernelFn hybrid_kernel_for(int dtype, int m) {
-  if (dtype == CSAHCA_BF16)
-    return m == 8 ? csa_hybrid_kernel<bf16, 128, 8> : m == 32 ? csa_hybrid_kernel<bf16, 128, 32>
-                                                               : csa_hybrid_kernel<bf16, 128, 0>;
-  return m == 8 ? csa_hybrid_kernel<f16, 128, 8> : m == 32 ? csa_hybrid_kernel<f16, 128, 32>
-                                                            : csa_hybrid_kernel<f16, 128, 0>;
+  return dtype == CSAHCA_BF16 ? hybrid_kernel_pick<bf16>(m) : hybrid_kernel_pick<f16>(m);
 }
 
 // Workgroups of kernel `fn` (kStepThreads threads, `lds` bytes of dynamic LDS)
@@ -1080,7 +1107,8 @@ int decode_step_impl(const void* q, const void* k_cache, const void* v_cache, co
   };
   size_t lds = lds_for(P);
   if (k > 0 && k <= kStepMaxK && fused_dtype && fused_dim && aligned && ncu > 0 && lds <= kStepLds) {
-    const int m = topk_regs_for(num_chunks, k);
+    const bool fine = head_dim == 128 && (dtype == CSAHCA_BF16 || dtype == CSAHCA_F16);
+    const int m = topk_regs_for(num_chunks, k, fine);
     const bool hyb = hybrid != nullptr && head_dim == 128 && pos_dev == nullptr &&
                      (dtype == CSAHCA_BF16 || dtype == CSAHCA_F16);
     const HybridKernelFn hfn = hyb ? hybrid_kernel_for(dtype, m) : nullptr;

@@ -72,3 +72,30 @@ def test_step_with_a_device_count(count):
     full = np.full((1, H, k), -1, dtype=np.int64)
     full[..., :min(k, count)] = want
     assert np.array_equal(idx.cpu().numpy(), full)
+
+
+@pytest.mark.parametrize("kind", ["random", "ties", "rising", "strided"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("C,k", [(1, 1), (63, 32), (64, 8), (127, 9), (128, 40), (129, 8), (512, 32), (513, 8),
+                                 (1023, 32), (1024, 9), (1025, 8)])
+def test_register_sizes_of_the_step(kind, dtype, C, k):
+    """head_dim 128 in 16 bits: at the edges of 2, 8, 16 and 32 keys per lane,
+    by the host's count, by the device's, and beside the HCA pass."""
+    H, D, chunk = 2, 128, 2
+    summ = _summary(_values(kind, H, C), D)
+    q = torch.zeros(1, H, D)
+    q[..., 0] = 1.0
+    q = q.to(dtype)
+    want, _ = oracle.select_topk(q, summ, k)
+    g = torch.Generator(device=DEV).manual_seed(C)
+    kc, vc = (torch.randn(1, H, C * chunk, D, generator=g, device=DEV).to(dtype) for _ in range(2))
+    qd, sd = q.to(DEV), summ.to(DEV)
+    out, idx = native.csa_decode_step(qd, kc, vc, sd, chunk, k)
+    assert np.array_equal(idx.cpu().numpy(), want)
+    n = torch.tensor([C], dtype=torch.int32, device=DEV)
+    _, idx = native.csa_decode_step_dev(qd, kc, vc, sd, n, chunk, k)
+    assert np.array_equal(idx.cpu().numpy(), want)
+    hyb = native.hybrid_decode_forward(qd, kc, vc, csa_chunk_size=chunk, csa_top_k=k, hca_chunk_size=chunk,
+                                       csa_weight=1.0, summary=sd)
+    diff = np.abs(hyb.double().cpu().numpy() - out.double().cpu().numpy())
+    assert np.all(diff <= 2e-2 + 1e-2 * np.abs(out.double().cpu().numpy()))
