@@ -54,7 +54,7 @@ __global__ __launch_bounds__(64) void csa_attend_vec_kernel(
   const IdxT* __restrict__ ib = idx + bh * top_k;
   const int total = top_k * chunk;
   const int s0 = t * tile;
-  const int s1 = min(s0 + tile, total);
+  const int s1 = s0 + min(tile, total - s0);  // (s0 + tile may be past int32)
   auto get_id = [&](int cs) { return ib[cs]; };
   auto tok_of = [&](int s, int64_t& tok) {
     return slot_token_of(get_id, s, chunk, chunk_shift, seq_len, tok);
@@ -111,7 +111,7 @@ __global__ __launch_bounds__(64) void csa_attend_generic_kernel(
   auto get_id = [&](int cs) { return ib[cs]; };
   const int total = top_k * chunk;
   const int s0 = t * tile;
-  const int s1 = min(s0 + tile, total);
+  const int s1 = s0 + min(tile, total - s0);  // (s0 + tile may be past int32)
   float m = -INFINITY, l = 0.f;
   // kGenericRows slots per batch: their chunk ids, then their K and V rows,
   // are each requested unconditionally as one batch (slots past the tile

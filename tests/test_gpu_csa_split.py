@@ -40,3 +40,20 @@ def test_split_matches_oracle(B, H, S, D, chunk, k, tile, dtype):
     atol, rtol = (2e-2, 1e-2) if dtype in (torch.bfloat16, torch.float16) else (1e-4, 1e-4)
     diff = np.abs(got.double().cpu().numpy() - ref)
     assert np.all(diff <= atol + rtol * np.abs(ref)), f"max_abs={diff.max():.3e}"
+
+
+def test_split_near_int32_slots():
+    """2^31 - 16384 slots: the last of 8192 tiles of 262144 would end past int32.
+    Only the last 8 chunks, all in that tile, hold an id."""
+    chunk, k, S, D = 16384, 131071, 32768, 64
+    g = torch.Generator().manual_seed(7)
+    q = torch.randn(1, 1, D, generator=g).to(torch.bfloat16)
+    kc = torch.randn(1, 1, S, D, generator=g).to(torch.bfloat16)
+    vc = torch.randn(1, 1, S, D, generator=g).to(torch.bfloat16) + 1.0
+    idx = torch.full((1, 1, k), -1, dtype=torch.int32)
+    idx[..., -8:] = 1
+    # (the same chunk 8 times: the softmax is that of the chunk once)
+    ref = oracle.csa_attend(q, kc, vc, torch.ones(1, 1, 1, dtype=torch.int32), chunk, prob_dtype=oracle.F32)
+    got = native.csa_decode_forward_tiled(q.to(DEV), kc.to(DEV), vc.to(DEV), idx.to(DEV), chunk, 128)
+    diff = np.abs(got.double().cpu().numpy() - ref)
+    assert np.all(diff <= 2e-2 + 1e-2 * np.abs(ref)), f"max_abs={diff.max():.3e}"
