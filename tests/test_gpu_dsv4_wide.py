@@ -140,3 +140,33 @@ def test_wide_kernel_decodes_every_code_exactly():
                                            page_size=64, softmax_scale=SCALE)
     got = out.double().cpu().numpy()
     assert np.array_equal(got, torch.from_numpy(np.asarray(want)).to(torch.bfloat16).double().numpy())
+
+
+def relative_error(got, ref):
+    return np.linalg.norm(got.double().cpu().numpy() - ref) / np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("q_scale,nats", [(1.0, 0.0), (2.0, 0.0), (4.0, 0.0), (1.0, 4.0), (1.0, 8.0), (1.0, 12.0),
+                                          (1.0, 20.0)])
+def test_wide_kernel_is_as_exact_as_the_kernel_it_stands_in_for(monkeypatch, q_scale, nats):
+    """Error against 64 bits (relative norm over 131072 values) of flat and of
+    peaked scores: one key past the first round `nats` above the rest weighs
+    nearly everything.  Not above the per-query kernel's, whose maximum moves:
+    3% for the spread of two independent sets of roundings, 1e-5 where both
+    outputs are nearly the key itself."""
+    c = make_dsv4_case(compress_ratio=0, num_queries=4, heads=64, num_tokens=640, top_k=640, page_size=64,
+                       full_lengths=True, seed=11, pack=False, device="cpu")
+    c.token_indices = torch.arange(640, dtype=torch.int32).repeat(4, 1)
+    c.q = (c.q.float() * q_scale).to(torch.bfloat16)
+    if nats:
+        c.q[:, :, 500] = 8.0  # a bf16 dim of the latent that only row 300 has
+        c.k_tokens[:, 500] = 0.0
+        c.k_tokens[300, 500] = nats * math.sqrt(512) / 8.0
+    c.cache = pack_dsv4_cache(c.k_tokens, page_size=64)
+    ref = oracle_out(c)
+    wide = relative_error(gpu_out(c), ref)
+    monkeypatch.setenv("CSAHCA_DSV4_WIDE", "0")
+    monkeypatch.setenv("CSAHCA_DSV4_QUERY", "1")
+    other = relative_error(gpu_out(c), ref)
+    print(f"q x {q_scale}, {nats} nats: wide {wide:.6f}, per-query {other:.6f}")
+    assert wide <= 1.03 * other + 1e-5
