@@ -1826,12 +1826,6 @@ __global__ __launch_bounds__(kWideWaves * kWave, 1) void dsv4_wide_kernel(const 
       for (int k = 0; k < 8; ++k) chunk_store(chunk_load(w, k), sc, k, b, std::true_type{});
     }
   };
-  // A row's scale bytes hold a 255: high bits of the bytes equal to it (the
-  // pad byte may count: no harm).
-  auto bytes_255 = [&](const uint2& sc) -> uint32_t {
-    return ((((sc.x & 0x7f7f7f7fu) + 0x01010101u) & sc.x) | (((sc.y & 0x7f7f7f7fu) + 0x01010101u) & sc.y)) & 0x80808080u;
-  };
-
   f32x16_t o[2][4];  // O^T[dims 128 wave + 32 db ..][heads 32 hb + l32]
   float m = -INFINITY, l = 0.f;  // head 32 hh + l32; l: this lane's slots only
   uint4 qb[32];                  // query operand: head 32 hh + l32, dims 16 t + 8 hl .. +7 of step t
@@ -1859,7 +1853,7 @@ __global__ __launch_bounds__(kWideWaves * kWave, 1) void dsv4_wide_kernel(const 
       idx_issue(2, loc);
       rows_at(1, loc1, nx);
       {
-        const bool any255 = __any((bytes_255(sc[0]) | bytes_255(sc[1])) != 0u);
+        const bool any255 = __any(has_scale_255(sc[0]) || has_scale_255(sc[1]));
 #pragma unroll
         for (int k = 0; k < 9; ++k) {
           chunk_store(c[k], sc, k, 0, std::false_type{});
@@ -1981,7 +1975,7 @@ __global__ __launch_bounds__(kWideWaves * kWave, 1) void dsv4_wide_kernel(const 
         for (int hb = 0; hb < 2; ++hb) p_read(0, hb);
 #pragma unroll
         for (int db = 0; db < 4; ++db) v_read(0, db);
-        const uint32_t s255 = bytes_255(sc[0]) | bytes_255(sc[1]);
+        const bool s255 = has_scale_255(sc[0]) || has_scale_255(sc[1]);
         // One step per 32 dims of 16 slots: two MFMAs, the reads of the step
         // four on, half a chunk of the next tile.
 #pragma unroll
@@ -2008,7 +2002,7 @@ __global__ __launch_bounds__(kWideWaves * kWave, 1) void dsv4_wide_kernel(const 
           }
           __builtin_amdgcn_sched_barrier(0);
         }
-        tile_finish(at, __any(s255 != 0u), b ^ 1);
+        tile_finish(at, __any(s255), b ^ 1);
         at = nx;
         lds_barrier();  // the next tile; P is free
       }

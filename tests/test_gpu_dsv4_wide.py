@@ -170,3 +170,50 @@ def test_wide_kernel_is_as_exact_as_the_kernel_it_stands_in_for(monkeypatch, q_s
     other = relative_error(gpu_out(c), ref)
     print(f"q x {q_scale}, {nats} nats: wide {wide:.6f}, per-query {other:.6f}")
     assert wide <= 1.03 * other + 1e-5
+
+
+def call_us(calls):
+    """Time of one call in us for each of `calls`, taken in turn: the least of
+    nine graph replays of eight calls."""
+    graphs = []
+    for call in calls:
+        stream = torch.cuda.Stream()
+        stream.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(stream):
+            call()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            for _ in range(8):
+                call()
+        graphs.append(graph)
+    us = [math.inf] * len(calls)
+    for _ in range(10):  # (the first replay of each warms up)
+        for i, graph in enumerate(graphs):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            graph.replay()
+            end.record()
+            torch.cuda.synchronize()
+            us[i] = min(us[i], start.elapsed_time(end) * 1e3 / 8)
+    return us
+
+
+def swa_call(c, cache, indices):
+    args = (c.q.to(DEV), cache.to(DEV), indices.to(DEV), c.topk_lengths.to(DEV), c.attn_sink.to(DEV))
+    return lambda: extension.dsv4_swa_decode_forward(*args, c.page_size, SCALE)
+
+
+def test_wide_kernel_pad_byte_is_not_a_scale():
+    """The eighth scale byte of a token holds whatever the cache's memory did:
+    0xFF there neither changes the output nor sends the tiles through the
+    general decode (1.3 times the time)."""
+    c = make_dsv4_case(compress_ratio=0, num_queries=64, heads=64, num_tokens=4096, top_k=640, page_size=64,
+                       full_lengths=True, seed=13, device="cpu")
+    padded = c.cache.clone()
+    for slot in range(64):
+        padded[:, 64 * 576 + 8 * slot + 7] = 255
+    plain, pad = swa_call(c, c.cache, c.token_indices), swa_call(c, padded, c.token_indices)
+    assert torch.equal(plain(), pad())
+    t_plain, t_pad = call_us([plain, pad])
+    assert t_pad < 1.12 * t_plain, f"{t_pad:.2f} us with pad bytes of 255, {t_plain:.2f} without"
