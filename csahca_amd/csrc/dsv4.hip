@@ -1568,7 +1568,8 @@ __global__ __launch_bounds__(NW * kWave) void dsv4_onepass_kernel(const int32_t*
 //     in registers) against 32 slots (half w / 2) with
 //     v_mfma_f32_32x32x16_bf16: S^T[slot][head], lane l = head l % 32; the
 //     addresses of the rows two rounds on are formed between the MFMAs.
-//   * Softmax against a fixed reference: the maximum m of the first round.
+//   * Softmax against a fixed reference: the maximum m of the first round that
+//     holds a row (skipped slots may fill whole rounds before it).
 //     p = 2^(x - m) may exceed 1 later on; fp32 and bf16 hold it at the same
 //     relative precision up to 2^127, so the accumulators are never rescaled
 //     and no branch surrounds them (a rescale under a branch moved all 128 out
@@ -1607,7 +1608,7 @@ struct WideShared {
   float mx[2][kWideHeads];        // per slot half: maxima, then sums
   float m[kWideHeads];            // the reference maxima
   uint8_t ok[2][kWideSlots];      // per tile: the slot holds a row
-  uint32_t full[2][kWideWaves];   // per tile and loading wavefront: all its 16 slots do
+  uint32_t full[2][kWideWaves];   // per tile and loading wavefront, of its 16 slots: 2 if any does, 3 if all do
   uint32_t flag[kWideWaves];
 };
 static_assert(sizeof(WideShared) <= 160 * 1024, "LDS of one workgroup");
@@ -1814,8 +1815,8 @@ __global__ __launch_bounds__(kWideWaves * kWave, 1) void dsv4_wide_kernel(const 
   // Which slots of the stored rows hold one, and (rare: a scale byte of 255)
   // their e4m3 chunks once more, through the general decode.
   auto tile_finish = [&](const Rows& w, bool any255, int b) {
-    const bool full = __all(w.ok[0] && w.ok[1]);
-    if (lane == 0) sm.full[b][wave] = full ? 1u : 0u;
+    const bool full = __all(w.ok[0] && w.ok[1]), any = __any(w.ok[0] || w.ok[1]);
+    if (lane == 0) sm.full[b][wave] = full ? 3u : any ? 2u : 0u;
     if (!full && c8 == 0) {
       sm.ok[b][16 * wave + r8] = w.ok[0];
       sm.ok[b][16 * wave + r8 + 8] = w.ok[1];
@@ -1839,6 +1840,7 @@ __global__ __launch_bounds__(kWideWaves * kWave, 1) void dsv4_wide_kernel(const 
     for (int i = 0; i < 16; ++i)
       *reinterpret_cast<uint4*>(sm.tile[1] + (16 * wave + i) * kQRow + 8 * lane) = qs[i];
   }
+  bool seek = true;  // no reference yet
   for (int pass = 0;; ++pass) {
     float mrun = -INFINITY;  // this lane's largest score
     l = 0.f;
@@ -1887,7 +1889,7 @@ __global__ __launch_bounds__(kWideWaves * kWave, 1) void dsv4_wide_kernel(const 
         const int b = r & 1;
         // ---- QK: S^T of 32 slots x 32 heads; between the MFMAs the
         // addresses of the rows two rounds on and the indices of the next ----
-        const bool full = (sm.full[b][2 * sb] & sm.full[b][2 * sb + 1]) != 0u;
+        const bool full = (sm.full[b][2 * sb] & sm.full[b][2 * sb + 1] & 1u) != 0u;
         const uint16_t* krow = sm.tile[b] + (32 * sb + l32) * kQRow + 8 * hl;
         f32x16_t s;
 #pragma unroll
@@ -1920,7 +1922,7 @@ __global__ __launch_bounds__(kWideWaves * kWave, 1) void dsv4_wide_kernel(const 
         if (__builtin_amdgcn_readfirstlane(full) == 0) {  // absent or invalid slots: -inf
 #pragma unroll
           for (int w = 0; w < 2; ++w) {
-            const bool wf = sm.full[b][2 * sb + w] != 0u;
+            const bool wf = (sm.full[b][2 * sb + w] & 1u) != 0u;
 #pragma unroll
             for (int i = 8 * w; i < 8 * w + 8; ++i)
               x[i] = (wf || sm.ok[b][32 * sb + 8 * (i / 4) + 4 * hl + i % 4]) ? x[i] : -INFINITY;
@@ -1931,11 +1933,14 @@ __global__ __launch_bounds__(kWideWaves * kWave, 1) void dsv4_wide_kernel(const 
         for (int i = 1; i < 15; i += 2) mw = fmaxf(fmaxf(mw, x[i]), x[i + 1]);
         mw = fmaxf(mw, x[15]);
         mrun = fmaxf(mrun, mw);
-        if (r == 0 && pass == 0) {  // the reference: the first round's maximum of each head
+        if (seek) {  // the reference: each head's maximum of the first round that holds a row
           mw = fmaxf(mw, __uint_as_float(lane_xor<32>(__float_as_uint(mw), lane)));
           if (hl == 0) sm.mx[sb][32 * hh + l32] = mw;
           lds_barrier();
           m = fmaxf(sm.mx[0][32 * hh + l32], sm.mx[1][32 * hh + l32]);
+          // (the same in every wavefront)
+          seek = __builtin_amdgcn_readfirstlane(
+                     static_cast<int>(sm.full[b][0] | sm.full[b][1] | sm.full[b][2] | sm.full[b][3])) == 0;
         }
         // ---- P rows: masked scores are -inf and give 0 (with no finite
         // reference, against 0) ----
@@ -2035,6 +2040,7 @@ __global__ __launch_bounds__(kWideWaves * kWave, 1) void dsv4_wide_kernel(const 
     if (__builtin_amdgcn_readfirstlane(static_cast<int>(sm.flag[0] | sm.flag[1] | sm.flag[2] | sm.flag[3])) == 0)
       break;  // workgroup-uniform; at most two passes
     m = mrun;
+    seek = false;
   }
   if (hl == 0) {
     sm.mx[sb][32 * hh + l32] = l;
