@@ -2321,20 +2321,30 @@ bool use_onepass(int64_t total_slots) {
 }
 
 // The wide kernel (64 heads and the whole list in one workgroup) takes a call
-// with more than 16 heads and a list of more than 256 slots whose (query, 16
-// heads) pairs come to half a workgroup of the other kernels per CU or more:
-// those fetch and dequantise every row once per 16 heads and dim part, and run
-// in waves of one workgroup per CU.  Measured per call (graph period, us)
-// against the per-query kernel, H 64, 384 / 640 slots: nq 32 21.1 / 32.8
-// against 21.3 / 29.4, nq 64 23.2 / 35.2 against 21.7 / 30.0, nq 256 89.1 /
-// 138.5 against 28.5 / 39.5.  With 16 heads or fewer three quarters of its MFMA
-// work would be padding (nq 256, 192 slots 15.7 against 17.6).
-// Shorter lists stay with the one-pass kernel, though the wide one is faster
-// there from 256 pairs (nq 80 18.4 against 13.6, nq 256 44.4 against 17.9 us at
-// 128 slots): the one-pass kernel rounds probabilities against the list's own
-// maximum, so that the largest is exact, the wide one against a reference fixed
-// before, and its error against 64 bits is 3% larger (relative norm 0.00219
-// against 0.00213).  Against the per-query kernel the two are equal (0.00214).
+// with more than 16 heads and a list of more than 256 slots, by its (query, 16
+// heads) pairs: the other kernels fetch and dequantise every row once per pair,
+// a workgroup per pair (two or four, by dims, where that many fit).
+//   * More pairs than CUs: they run in waves there, the wide kernel is faster
+//     at every length (nq 128 x H 64, 257 / 384 / 640 / 1024 slots: 23.4 / 25.0
+//     / 33.3 / 46.1 us a call against 38.4 / 46.8 / 69.5 / 106.0).
+//   * Fewer, down to half: one wave there, and a round of 64 slots takes the
+//     wide kernel 2.05 us against 2.9, so it is behind up to the length where
+//     that makes up for its 8 us around the rounds and for a last round that
+//     is not full (its masks: 1.2 us).  nq 32 x H 64, 320 / 352 / 384 / 448 /
+//     512 slots: 20.2 / 23.4 / 22.1 / 24.4 / 26.3 against 19.4 / 21.6 / 22.1 /
+//     25.3 / 28.1; nq 40 (160 pairs, two dim parts no longer fit): 20.3 / 23.5 /
+//     22.3 / 24.5 / 26.7 against 20.9 / 23.2 / 23.9 / 26.8 / 29.7; nq 64 20.5 /
+//     23.9 / 22.6 / 24.8 / 27.0 against 21.3 / 23.9 / 24.5 / 27.8 / 30.8; the
+//     same line at H 24, 32, 80 and 128.
+// With 16 heads or fewer three quarters of its MFMA work would be padding (nq
+// 256, 192 slots 15.7 against 17.6).
+// Lists of up to 256 slots stay with the one-pass kernel, though the wide one
+// is faster there from 256 pairs (nq 80 18.4 against 13.6, nq 256 44.4 against
+// 17.9 us at 128 slots): the one-pass kernel rounds probabilities against the
+// list's own maximum, so that the largest is exact, the wide one against a
+// reference fixed before, and its error against 64 bits is larger (relative
+// norm at 192 slots 0.00218 against 0.00213, q x 2 0.00200 against 0.00188).
+// Against the per-query kernel it is not (0.00214 / 0.00214, 0.00208 / 0.00224).
 // CSAHCA_DSV4_WIDE=0 / 1 forces the choice; CSAHCA_DSV4_QUERY=0 / 1, which
 // forces a kernel of the longer lists, turns it off (all read per call).
 bool use_wide(int64_t nq, int64_t heads, int64_t total_slots) {
@@ -2344,6 +2354,7 @@ bool use_wide(int64_t nq, int64_t heads, int64_t total_slots) {
   const int ncu = device_cu_count();
   const int64_t pairs = ceil_div(nq, 8) * 8 * ceil_div(heads, kQHeads);
   if (heads <= kQHeads || ncu <= 0 || total_slots <= kOpMaxSlots || 2 * pairs < ncu) return false;
+  if (pairs <= ncu && total_slots < (8 * pairs >= 5 * ncu && total_slots % kWideSlots == 0 ? 320 : 384)) return false;
   const char* f = env_switch("CSAHCA_DSV4_QUERY");
   return !(f && (f[0] == '0' || f[0] == '1'));
 }

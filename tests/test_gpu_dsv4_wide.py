@@ -234,3 +234,35 @@ def test_wide_kernel_skipped_slots_first(skipped):
     c.q, c.token_indices, c.topk_lengths = c.q[:4], indices[:4], c.topk_lengths[:4]
     assert_close(late()[:4], oracle_out(c))
     assert t_late < 1.3 * t_full, f"{t_late:.2f} us with {skipped} slots skipped, {t_full:.2f} without"
+
+
+def kernels_of(call):
+    with native.profile_launches() as p:
+        call()
+        torch.cuda.synchronize()
+    return set(p.results)
+
+
+@pytest.mark.parametrize("nq,heads,slots,wide", [
+    (72, 64, 257, True),    # more (query, 16 heads) pairs than CUs
+    (72, 64, 256, False),   # the longest list of the one-pass kernel
+    (64, 64, 304, False),   # 256 pairs
+    (64, 64, 320, True),    # whole rounds
+    (64, 64, 352, False),
+    (64, 64, 384, True),
+    (32, 64, 320, False),   # 128 pairs
+    (32, 64, 383, False),
+    (32, 64, 384, True),
+    (256, 16, 640, False),  # 16 heads: three quarters padding
+])
+def test_wide_kernel_takes_its_calls(monkeypatch, nq, heads, slots, wide):
+    """The rule by itself, no switch set (on a device of 256 CUs)."""
+    monkeypatch.delenv("CSAHCA_DSV4_WIDE")
+    assert torch.cuda.get_device_properties(0).multi_processor_count == 256
+    c = make_dsv4_case(compress_ratio=0, num_queries=nq, heads=heads, num_tokens=700, top_k=slots, page_size=64,
+                       seed=slots, device="cpu")
+    call = swa_call(c, c.cache, c.token_indices)
+    assert ("dsv4_wide_kernel" in kernels_of(call)) == wide
+    out = call()[:2]
+    c.q, c.token_indices, c.topk_lengths = c.q[:2], c.token_indices[:2], c.topk_lengths[:2]
+    assert_close(out, oracle_out(c))
