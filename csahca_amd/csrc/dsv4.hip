@@ -2323,11 +2323,13 @@ bool use_onepass(int64_t total_slots) {
 // The wide kernel (64 heads and the whole list in one workgroup) takes a call
 // with more than 16 heads and a list of more than 256 slots, by its (query, 16
 // heads) pairs: the other kernels fetch and dequantise every row once per pair,
-// a workgroup per pair (two or four, by dims, where that many fit).
+// a workgroup per pair (two or four, by dims, where that many fit).  Pairs of
+// real queries: the grid's rows of eight made 128 of the 16 pairs of 1 query x
+// 256 heads (640 slots 15.9 us on the split kernel, 30.0 here).
 //   * More pairs than CUs: they run in waves there, the wide kernel is faster
 //     at every length (nq 128 x H 64, 257 / 384 / 640 / 1024 slots: 23.4 / 25.0
 //     / 33.3 / 46.1 us a call against 38.4 / 46.8 / 69.5 / 106.0).
-//   * Fewer, down to half: one wave there, and a round of 64 slots takes the
+//   * Fewer, down to a quarter: one wave there, and a round of 64 slots takes the
 //     wide kernel 2.05 us against 2.9, so it is behind up to the length where
 //     that makes up for its 8 us around the rounds and for a last round that
 //     is not full (its masks: 1.2 us).  nq 32 x H 64, 320 / 352 / 384 / 448 /
@@ -2335,7 +2337,9 @@ bool use_onepass(int64_t total_slots) {
 //     25.3 / 28.1; nq 40 (160 pairs, two dim parts no longer fit): 20.3 / 23.5 /
 //     22.3 / 24.5 / 26.7 against 20.9 / 23.2 / 23.9 / 26.8 / 29.7; nq 64 20.5 /
 //     23.9 / 22.6 / 24.8 / 27.0 against 21.3 / 23.9 / 24.5 / 27.8 / 30.8; the
-//     same line at H 24, 32, 80 and 128.
+//     same line at H 24, 32, 80 and 128.  Below half, nq 24 x H 64, 384 / 448 /
+//     512: 22.2 / 24.3 / 26.3 against 22.0 / 24.9 / 27.9.
+//   * Fewer still take the split kernel.
 // With 16 heads or fewer three quarters of its MFMA work would be padding (nq
 // 256, 192 slots 15.7 against 17.6).
 // Lists of up to 256 slots stay with the one-pass kernel, though the wide one
@@ -2352,9 +2356,13 @@ bool use_wide(int64_t nq, int64_t heads, int64_t total_slots) {
   const char* e = env_switch("CSAHCA_DSV4_WIDE");
   if (e && (e[0] == '0' || e[0] == '1') && e[1] == 0) return e[0] == '1';
   const int ncu = device_cu_count();
-  const int64_t pairs = ceil_div(nq, 8) * 8 * ceil_div(heads, kQHeads);
-  if (heads <= kQHeads || ncu <= 0 || total_slots <= kOpMaxSlots || 2 * pairs < ncu) return false;
-  if (pairs <= ncu && total_slots < (8 * pairs >= 5 * ncu && total_slots % kWideSlots == 0 ? 320 : 384)) return false;
+  const int64_t pairs = nq * ceil_div(heads, kQHeads);
+  if (heads <= kQHeads || ncu <= 0 || total_slots <= kOpMaxSlots || 4 * pairs < ncu) return false;
+  if (pairs <= ncu) {
+    const bool whole = total_slots % kWideSlots == 0;
+    const int64_t line = 8 * pairs >= 5 * ncu && whole ? 320 : 2 * pairs >= ncu ? 384 : 512;
+    if (total_slots < line) return false;
+  }
   const char* f = env_switch("CSAHCA_DSV4_QUERY");
   return !(f && (f[0] == '0' || f[0] == '1'));
 }

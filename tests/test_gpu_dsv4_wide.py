@@ -253,6 +253,13 @@ def kernels_of(call):
     (32, 64, 320, False),   # 128 pairs
     (32, 64, 383, False),
     (32, 64, 384, True),
+    (31, 64, 384, False),   # 124 pairs
+    (31, 64, 512, True),
+    (16, 64, 512, True),    # 64 pairs
+    (15, 64, 512, False),
+    (1, 256, 384, False),   # 16 pairs, in a grid of 128
+    (1, 256, 640, False),
+    (4, 256, 640, True),    # 64 pairs
     (256, 16, 640, False),  # 16 heads: three quarters padding
 ])
 def test_wide_kernel_takes_its_calls(monkeypatch, nq, heads, slots, wide):
