@@ -17,6 +17,7 @@
 //                        independent of each other.
 // csa_step.hip fuses 2-5 into one launch.  All offsets are 64-bit.
 #include "csa_device.hpp"
+#include "dispatch.hpp"
 
 #include <algorithm>
 #include <climits>
@@ -246,7 +247,7 @@ __global__ __launch_bounds__(256) void csa_merge_cols_kernel(const float* __rest
   }
 }
 
-// The same merge over any number of partials (split_tile gives more than
+// The same merge over any number of partials (csa_split_tile gives more than
 // kMergeColTiles only to heads with long selections): the maximum over all
 // tiles first, then kMergePass tiles at a time -- weights once per workgroup
 // into LDS, then every thread its column of the pass's tiles g, g + 8, ...,
@@ -512,33 +513,10 @@ size_t decode_ws_bytes(int64_t bh, int64_t D, int64_t tiles) {
   return ml_al + static_cast<size_t>(bh * tiles * D) * sizeof(float);
 }
 
-// Slots per wavefront of the split: the caller's tile, or the smallest multiple
-// of it that
-//   * fills one batch of row loads of the attend kernel (16 slots at 16-bit
-//     head_dim 128, 32 at 64, 4 in the generic kernel; a smaller tile re-reads
-//     its last row);
-//   * leaves a head at most 64 tiles, the one-round-trip merge, as long as that
-//     makes tiles of at most 128 slots;
-//   * leaves the call at most 8192 wavefronts (32 per CU): more only write and
-//     merge more partials.
-// A tile is a hint for the split, and the partials of several of the caller's
-// tiles are one partial of their union, so the workspace the caller sized for
-// its own tile holds them.  Measured (graph period, us, tile 8 as called /
-// split chosen): B1 H8 D128 top-8 5.31 / 5.06, top-32 49.3 / 7.3; B8 top-16
-// 16.4 / 10.3, top-32 60.6 / 15.3; B32 top-32 104.7 / 56.7; B4 H12 D64 f16
-// 480 slots 7.3 / 6.4; f32 D256 512 slots 9.4 (kept at 8).
-int64_t split_tile(int64_t tile, int64_t total, int64_t bh, int64_t D, int64_t esz) {
-  const bool vec = (D == 64 || D == 128 || D == 256 || D == 512) && D * esz / 16 <= kWave;
-  const int64_t batch = vec ? 4 * (kWave / (D * esz / 16)) : 4;
-  const int64_t want = std::max({batch, std::min<int64_t>(ceil_div(total, kMergeColTiles), 128), ceil_div(total * bh, 8192)});
-  const int64_t t = tile >= want ? tile : ceil_div(want, tile) * tile;
-  return std::min<int64_t>(t, std::max<int64_t>(total, 1));
-}
-
 template <typename T, typename IdxT>
 int launch_attend(const void* q, const void* k, const void* v, const void* idx, float* part_ml,
                   float* part_acc, int64_t bh, int64_t S, int64_t D, int top_k, int chunk,
-                  int tile, int num_tiles, hipStream_t stream) {
+                  int tile, int num_tiles, bool vec, hipStream_t stream) {
   const float qscale = kLog2e / sqrtf(static_cast<float>(D));
   const int cshift = chunk_shift_of(chunk);
   const dim3 grid(static_cast<uint32_t>(bh * num_tiles));
@@ -547,10 +525,8 @@ int launch_attend(const void* q, const void* k, const void* v, const void* idx, 
   const T* vp = static_cast<const T*>(v);
   const IdxT* ip = static_cast<const IdxT*>(idx);
   constexpr int VEC = Vec16<T>::N;
-  const bool aligned = (reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) |
-                        reinterpret_cast<uintptr_t>(v)) % 16 == 0;
 #define CSAHCA_ATTEND_VEC(DD)                                                                  \
-  if (aligned && D == DD && (DD / VEC) <= kWave) {                                           \
+  if (vec && D == DD && (DD / VEC) <= kWave) {                                               \
     return launch("csa_attend_vec_kernel",                                                   \
                   csa_attend_vec_kernel<T, IdxT, (DD / VEC <= kWave ? DD : VEC), 4>, grid,   \
                   dim3(kWave), 0, stream, ip, S, kp, vp, qp, num_tiles, top_k, tile, chunk,    \
@@ -601,7 +577,10 @@ int csa_decode_impl(const void* q, const void* k, const void* v, const void* idx
   if (workspace == nullptr || workspace_bytes < need)
     return fail(CSAHCA_ERR_WORKSPACE, "workspace too small for csa decode");
   const int64_t esz = dtype == CSAHCA_F64 ? 8 : dtype == CSAHCA_F32 ? 4 : 2;
-  tile = split_tile(tile, total, bh, D, esz);
+  // (the vectorised kernel: 16-byte rows and loads, a row in at most a wavefront)
+  const bool vec = (D == 64 || D == 128 || D == 256 || D == 512) && D * esz / 16 <= kWave &&
+                   (reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v)) % 16 == 0;
+  tile = csa_split_tile(tile, total, bh, D, esz, vec);
   const int64_t tiles = std::max<int64_t>(1, ceil_div(total, tile));  // <= asked
   float* part_ml = static_cast<float*>(workspace);
   const size_t ml = static_cast<size_t>(bh * tiles * 2) * sizeof(float);
@@ -617,10 +596,10 @@ int csa_decode_impl(const void* q, const void* k, const void* v, const void* idx
     int rc = index_dtype == CSAHCA_I32
                  ? launch_attend<T, int32_t>(q, k_ok, v_ok, idx_ok, part_ml, part_acc, bh, S, D,
                                              static_cast<int>(top_k), static_cast<int>(chunk), tl,
-                                             static_cast<int>(tiles), stream)
+                                             static_cast<int>(tiles), vec, stream)
                  : launch_attend<T, int64_t>(q, k_ok, v_ok, idx_ok, part_ml, part_acc, bh, S, D,
                                              static_cast<int>(top_k), static_cast<int>(chunk), tl,
-                                             static_cast<int>(tiles), stream);
+                                             static_cast<int>(tiles), vec, stream);
     if (rc != CSAHCA_OK) return rc;
     if (tiles <= kMergeColTiles) {
       const int64_t cbs = ceil_div(D, kMergeCols);

@@ -1,0 +1,82 @@
+"""The rules on sizes that choose a launch (csahca_amd/csrc/dispatch.hpp), built
+alone with the host compiler."""
+import ctypes
+import subprocess
+from pathlib import Path
+
+import pytest
+
+CSRC = Path(__file__).resolve().parents[1] / "csahca_amd" / "csrc"
+SHIM = r"""
+#include "dispatch.hpp"
+extern "C" {
+int64_t split_tile(int64_t tile, int64_t total, int64_t bh, int64_t D, int64_t esz, int vec) {
+  return csahca::csa_split_tile(tile, total, bh, D, esz, vec != 0);
+}
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    d = tmp_path_factory.mktemp("rules")
+    (d / "shim.cpp").write_text(SHIM)
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-O1", "-shared", "-fPIC", f"-I{CSRC}", "-o",
+                    str(d / "rules.so"), str(d / "shim.cpp")], check=True)
+    lib = ctypes.CDLL(str(d / "rules.so"))
+    lib.split_tile.restype = ctypes.c_int64
+    lib.split_tile.argtypes = [ctypes.c_int64] * 5 + [ctypes.c_int]
+    return lib
+
+
+@pytest.mark.parametrize("tile,total,bh,D,esz,want", [
+    (16, 3200, 8, 40, 2, 16),     # tiles of 64 took 1.43 times as long
+    (32, 3200, 8, 96, 2, 32),     # 1.24
+    (32, 3200, 256, 40, 2, 32),   # 1.16
+    (64, 3200, 256, 96, 2, 64),   # 1.15
+    (16, 800, 256, 96, 2, 16),    # 1.08
+    (8, 1600, 8, 96, 2, 16),
+    (8, 800, 8, 96, 2, 16),
+    (4, 400, 32, 96, 2, 8),
+    (4, 200, 8, 96, 2, 4),
+    (1, 64, 1, 96, 2, 4),
+    (3, 64, 1, 96, 2, 6),
+    (5, 3200, 8, 96, 2, 15),
+    (12, 3200, 8, 96, 2, 12),
+    (8, 3200, 256, 96, 2, 32),    # 300 MiB of rows of 192 bytes
+    (16, 800, 256, 192, 2, 16),
+    (4, 256, 256, 192, 2, 8),
+    (4, 3200, 256, 192, 2, 64),   # 600 MiB of rows of 384: no limit
+    (4, 3200, 256, 320, 4, 100),  # rows of 1280
+    (4, 6400, 32, 320, 4, 100),
+    (64, 3200, 256, 192, 2, 64),
+])
+def test_generic_split_keeps_its_chain_short(rules, tile, total, bh, D, esz, want):
+    assert rules.split_tile(tile, total, bh, D, esz, 0) == want
+
+
+@pytest.mark.parametrize("tile,total,bh,D,esz,want", [
+    (8, 512, 8, 128, 2, 16),      # a batch of row loads
+    (8, 480, 48, 64, 2, 32),
+    (8, 512, 16, 256, 4, 8),
+    (8, 2048, 8, 128, 2, 32),     # 64 tiles a head
+    (8, 1024, 64, 128, 2, 16),
+    (5, 192, 6, 128, 2, 20),
+    (1, 16384, 1, 128, 2, 128),
+    (8, 2048, 256, 128, 2, 64),   # 8192 wavefronts
+])
+def test_vectorised_split(rules, tile, total, bh, D, esz, want):
+    assert rules.split_tile(tile, total, bh, D, esz, 1) == want
+
+
+@pytest.mark.parametrize("vec", [0, 1])
+def test_split_fits_the_callers_workspace(rules, vec):
+    """Never more tiles than the caller's own tile makes, never an empty tile."""
+    for tile in (1, 3, 5, 7, 8, 16, 33, 64, 128, 1000, 1 << 31):
+        for total in (0, 1, 4, 17, 64, 100, 3200, 16384, 2**31 - 16384, 2**31 - 1):
+            for bh in (1, 8, 256, 100000):
+                for D, esz in ((64, 2), (128, 2), (256, 4)):
+                    t = rules.split_tile(tile, total, bh, D, esz, vec)
+                    assert 1 <= t <= max(total, 1)
+                    assert t >= min(tile, max(total, 1))
+                    assert -(-total // t) <= max(1, -(-total // tile))

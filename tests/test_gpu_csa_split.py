@@ -19,9 +19,9 @@ DEV = "cuda"
     (1, 1, 8256, 64, 64, 129, 1, torch.float16),       # 65 tiles: one past the one-round-trip merge
     (1, 1, 132000, 64, 1000, 132, 7, torch.float16),   # 997 tiles of 133 slots
     (1, 1, 140000, 64, 1000, 140, 8, torch.bfloat16),  # 1094 tiles: two passes of weights
-    (2, 1, 9000, 96, 50, 180, 8, torch.bfloat16),      # generic kernel, 71 tiles; columns that are no multiple of 32
+    (2, 1, 9000, 96, 50, 180, 8, torch.bfloat16),      # generic kernel, 563 tiles; columns that are no multiple of 32
     (1, 2, 9216, 256, 48, 190, 3, torch.float32),      # 72 tiles of 129 slots
-    (1, 1, 9216, 100, 64, 144, 8, torch.float64),      # 72 tiles, 100 columns
+    (1, 1, 9216, 100, 64, 144, 8, torch.float64),      # generic kernel, 576 tiles, 100 columns
     (3, 2, 640, 128, 64, 3, 5, torch.bfloat16),        # 192 slots: tiles of 20 for the asked 5
     (1, 1, 64, 64, 16, 1, 3, torch.float16),           # 16 slots in one tile of at most 33
 ])
