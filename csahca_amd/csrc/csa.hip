@@ -643,7 +643,7 @@ int csa_select_launch(const void* q, const float* summary, int32_t* out_indices,
   });
   if (rc != CSAHCA_OK) return rc;
   // One wavefront with two keys per lane up to where 64 candidates hold the
-  // answer (see topk_regs_for); the workgroup otherwise.  Measured, 8 heads,
+  // answer (see csa_step_topk_regs); the workgroup otherwise.  Measured, 8 heads,
   // registers against block_topk, us a call with the scores: top-32 of 64,
   // 128, 256, 512: 4.5 / 5.1, 5.0 / 5.4, 5.7 / 5.3, 6.8 / 6.0; top-8 of 1024, 2048: 9.6
   // / 6.6, 14.4 / 8.3; top-40, 48 of 128: 5.2 / 5.4, 11.7 / 5.3.

@@ -428,30 +428,6 @@ __device__ __forceinline__ int32_t wave_top1(const uint32_t* keys, int C) {
   return static_cast<int32_t>(~static_cast<uint32_t>(c));
 }
 
-// Register-path size for the fused step's selection: keys per lane M (C <= 64
-// * M), or 0 for block_topk (k <= 64) or the radix select.  Kernels take M as a
-// template parameter so each instantiation carries exactly one of them.  The
-// register path fails where more than 64 keys reach its threshold, which of
-// independent keys 64 ln(64 / (64 - k)) do (44 for k = 32, 63 for 40, 89 for
-// 48), fewer of at most 2 per lane; the radix select behind it costs 6-24 us.
-// Measured, B1 H8 D128 chunk 16, registers against block_topk, us a step:
-// top-32 of 512, 1024, 2048: 8.5 / 9.4, 10.95 / 11.1, 12.5 / 13.0; top-40 of 64,
-// 128, 256: 9.3 / 10.0, 9.3 / 9.8, 16.1 / 9.8; top-64 of 64, 128, 512, 2048: 9.6 /
-// 10.2, 18.3 / 10.7, 21.4 / 11.5, 36.2 / 13.7.
-// The fewest keys per lane that hold C: `fine` where the kernels with 2 and 16
-// exist (head_dim 128 in 16 bits; bf16 us a step, top-8: 128 chunks with 8 and
-// with 2 7.92 / 7.59, 1024 with 32 and with 16 10.0 / 9.15).
-inline int topk_regs_for(int64_t C, int64_t k, bool fine) {
-  if (C > 64 && k > 40) return 0;
-  if (C > 128 && k > 32) return 0;
-  if (k > kWave) return 0;
-  if (fine && C <= 128) return 2;
-  if (C <= 512) return 8;
-  if (fine && C <= 1024) return 16;
-  if (C <= 2048) return 32;
-  return 0;
-}
-
 // Top-k with the declared order: the register path when M > 0 (falling back
 // when too many keys tie around its threshold), else the LDS radix select.
 template <int M, typename Out>

@@ -36,6 +36,7 @@
 // The workspace must be zero before the first launch and whenever the problem
 // shape (B*H, chunks, head_dim, top_k, chunk) changes.
 #include "csa_device.hpp"
+#include "dispatch.hpp"
 #include "hca_device.hpp"
 
 #include <algorithm>
@@ -1108,7 +1109,7 @@ int decode_step_impl(const void* q, const void* k_cache, const void* v_cache, co
   size_t lds = lds_for(P);
   if (k > 0 && k <= kStepMaxK && fused_dtype && fused_dim && aligned && ncu > 0 && lds <= kStepLds) {
     const bool fine = head_dim == 128 && (dtype == CSAHCA_BF16 || dtype == CSAHCA_F16);
-    const int m = topk_regs_for(num_chunks, k, fine);
+    const int m = csa_step_topk_regs(num_chunks, k, bh, fine);
     const bool hyb = hybrid != nullptr && head_dim == 128 && pos_dev == nullptr &&
                      (dtype == CSAHCA_BF16 || dtype == CSAHCA_F16);
     const HybridKernelFn hfn = hyb ? hybrid_kernel_for(dtype, m) : nullptr;

@@ -54,4 +54,31 @@ inline int64_t csa_split_tile(int64_t tile, int64_t total, int64_t bh, int64_t D
   return std::min<int64_t>(t, std::max<int64_t>(total, 1));
 }
 
+// Register-path size for the fused step's selection of k of C chunks: keys per
+// lane M (C <= 64 * M), or 0 for block_topk (k <= 64) or the radix select.
+// Kernels take M as a template parameter so each instantiation carries exactly
+// one of them.  The register path fails where more than 64 keys reach its
+// threshold, which of independent keys 64 ln(64 / (64 - k)) do (44 for k = 32,
+// 53 for 36, 63 for 40), fewer of few per lane; the radix select behind it costs
+// 6-20 us, and one head of the call that takes it costs the call that.  So the
+// line for more than 128 chunks is where a call of all its heads still rarely
+// fails.  Simulated, failures a head at k = 34 / 36 / 38 / 40: 256 chunks <1e-5 /
+// 9e-5 / 2.6e-3 / 2.7e-2, 512 chunks 5e-5 / 2.9e-3 / 2.6e-2 / 0.13, 2048 chunks
+// 1.1e-3 / 1.3e-2 / 7.9e-2 / 0.27.  Measured, B1 H8 D128 chunk 16, registers
+// (not failing) against block_topk, us a step: top-33 of 256, 512, 1024, 2048:
+// 9.4 / 10.1, 9.5 / 10.5, 11.6 / 11.7, 12.9 / 13.5; top-36 of 256, 512: 9.4 / 10.1,
+// 9.6 / 10.5; top-40 of 64, 128: 9.3 / 10.0, 9.3 / 9.8, and failing, of 384: 17.6 /
+// 10.5; top-64 of 64, 128, 512, 2048: 9.6 / 10.2, 18.3 / 10.7, 21.4 / 11.5, 36.2 /
+// 13.7.
+// The fewest keys per lane that hold C: `fine` where the kernels with 2 and 16
+// exist (head_dim 128 in 16 bits; bf16 us a step, top-8: 128 chunks with 8 and
+// with 2 7.92 / 7.59, 1024 with 32 and with 16 10.0 / 9.15).
+inline int csa_step_topk_regs(int64_t C, int64_t k, int64_t bh, bool fine) {
+  const int64_t most = C <= 64 ? 64 : C <= 128 ? 40 : (C <= 256 ? 36 : C <= 512 ? 34 : 32) + (bh <= 16 ? 2 : 0);
+  if (k > most || C > 2048) return 0;
+  if (fine && C <= 128) return 2;
+  if (C <= 512) return 8;
+  return fine && C <= 1024 ? 16 : 32;
+}
+
 }  // namespace csahca
