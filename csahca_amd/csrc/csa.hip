@@ -642,12 +642,7 @@ int csa_select_launch(const void* q, const float* summary, int32_t* out_indices,
                   static_cast<int>(D), scale);
   });
   if (rc != CSAHCA_OK) return rc;
-  // One wavefront with two keys per lane up to where 64 candidates hold the
-  // answer (see csa_step_topk_regs); the workgroup otherwise.  Measured, 8 heads,
-  // registers against block_topk, us a call with the scores: top-32 of 64,
-  // 128, 256, 512: 4.5 / 5.1, 5.0 / 5.4, 5.7 / 5.3, 6.8 / 6.0; top-8 of 1024, 2048: 9.6
-  // / 6.6, 14.4 / 8.3; top-40, 48 of 128: 5.2 / 5.4, 11.7 / 5.3.
-  const int regs = k <= kWave && (C <= kWave || (C <= 2 * kWave && k <= 40)) ? 2 : 0;
+  const int regs = csa_select_topk_regs(C, k);
   const size_t base =
       kCandBytes + (256 + 2 * static_cast<size_t>(k) + 1 + (regs ? 0 : kTopkListWords)) * sizeof(uint32_t);
   const bool in_lds = base + static_cast<size_t>(C) * sizeof(uint32_t) <= kLdsBudget;
@@ -656,6 +651,7 @@ int csa_select_launch(const void* q, const float* summary, int32_t* out_indices,
   const uint32_t* kp = keys;
   const int ki = static_cast<int>(k);
   switch (regs * 2 + (in_lds ? 1 : 0)) {
+    case 9: return launch("csa_topk_kernel", csa_topk_kernel<4, true>, grid, dim3(kWave), lds, stream, kp, out_indices, C, ki);
     case 5: return launch("csa_topk_kernel", csa_topk_kernel<2, true>, grid, dim3(kWave), lds, stream, kp, out_indices, C, ki);
     case 1: return launch("csa_topk_kernel", csa_topk_kernel<0, true>, grid, dim3(kTopkWaves * kWave), lds, stream, kp, out_indices, C, ki);
     default: return launch("csa_topk_kernel", csa_topk_kernel<0, false>, grid, dim3(kTopkWaves * kWave), lds, stream, kp, out_indices, C, ki);

@@ -81,4 +81,15 @@ inline int csa_step_topk_regs(int64_t C, int64_t k, int64_t bh, bool fine) {
   return fine && C <= 1024 ? 16 : 32;
 }
 
+// The same for the selection op: keys per lane of its one-wavefront kernel, or 0
+// for the workgroup's.  Measured, 8 heads, registers against block_topk, us a
+// call with the scores: top-32 of 64, 128: 4.5 / 5.1, 5.0 / 5.4; top-40, 48 of
+// 128: 5.2 / 5.4, 11.7 / 5.3; top-8 of 129, 160, 192: 4.94 / 5.32, 5.18 / 5.30,
+// 5.11 / 5.27; top-36 of 129, 192: 5.32 / 5.76, 5.56 / 5.72; top-16 level.
+inline int csa_select_topk_regs(int64_t C, int64_t k) {
+  if (C <= 64) return k <= 64 ? 2 : 0;
+  if (C <= 128) return k <= 40 ? 2 : 0;
+  return C <= 192 && k <= 36 ? 4 : 0;
+}
+
 }  // namespace csahca

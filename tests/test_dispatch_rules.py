@@ -13,6 +13,7 @@ extern "C" {
 int64_t split_tile(int64_t tile, int64_t total, int64_t bh, int64_t D, int64_t esz, int vec) {
   return csahca::csa_split_tile(tile, total, bh, D, esz, vec != 0);
 }
+int select_topk_regs(int64_t C, int64_t k) { return csahca::csa_select_topk_regs(C, k); }
 int step_topk_regs(int64_t C, int64_t k, int64_t bh, int fine) {
   return csahca::csa_step_topk_regs(C, k, bh, fine != 0);
 }
@@ -30,6 +31,7 @@ def rules(tmp_path_factory):
     lib.split_tile.restype = ctypes.c_int64
     lib.split_tile.argtypes = [ctypes.c_int64] * 5 + [ctypes.c_int]
     lib.step_topk_regs.argtypes = [ctypes.c_int64] * 3 + [ctypes.c_int]
+    lib.select_topk_regs.argtypes = [ctypes.c_int64] * 2
     return lib
 
 
@@ -105,3 +107,11 @@ def test_step_selection_registers_hold_every_key(rules):
         for fine in (0, 1):
             m = rules.step_topk_regs(C, 8, 8, fine)
             assert m in ((2, 8, 16, 32) if fine else (8, 32)) and 64 * m >= C
+
+
+@pytest.mark.parametrize("C,k,want", [
+    (1, 1, 2), (64, 64, 2), (64, 65, 0), (128, 40, 2), (128, 41, 0), (129, 1, 4), (192, 36, 4), (192, 37, 0), (193, 1, 0),
+])
+def test_selection_op_takes_registers_up_to_192_chunks(rules, C, k, want):
+    """129-192 chunks went to the workgroup's top-k, 2-6% slower a call."""
+    assert rules.select_topk_regs(C, k) == want

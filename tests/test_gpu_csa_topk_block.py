@@ -1,7 +1,8 @@
-"""Selection of at most 64 keys by all wavefronts of a workgroup (in the step
-where one wavefront's registers or candidates do not hold it), in the selection op and in the fused step: the oracle's indices and
-order exactly.  Keys are the first component of each summary row (q is its unit
-vector), so scores carry no rounding."""
+"""Selection of at most 64 keys, by one wavefront's registers and, where they or
+its candidates do not hold it, by all wavefronts of a workgroup, in the
+selection op and in the fused step: the oracle's indices and order exactly.
+Keys are the first component of each summary row (q is its unit vector), so
+scores carry no rounding."""
 import numpy as np
 import pytest
 import torch
@@ -36,7 +37,7 @@ def _values(kind, bh, C):
 @pytest.mark.parametrize("kind", ["random", "ties", "rising", "strided", "negative infinity"])
 @pytest.mark.parametrize("C,k", [(64, 64), (65, 40), (65, 41), (128, 40), (129, 33), (255, 33), (257, 64), (512, 41),
                                  (2048, 33), (2049, 1), (2303, 64), (2305, 8), (4096, 64), (6295, 14), (14003, 63), (20001, 64),
-                                 (2500, 65)])
+                                 (2500, 65), (129, 1), (192, 36), (192, 37), (256, 36), (512, 34)])
 def test_selection_and_step_match_the_oracle(kind, C, k):
     H, D, chunk = 3, 64, 2
     summ = _summary(_values(kind, H, C), D)
