@@ -92,4 +92,34 @@ inline int csa_select_topk_regs(int64_t C, int64_t k) {
   return C <= 192 && k <= 36 ? 4 : 0;
 }
 
+// Whether the hybrid op reads K once for the summaries and the HCA chunk pass
+// (`items` HCA chunks of hca_chunk rows over all heads).  A wavefront walks a
+// whole HCA chunk of one tensor, and is the longer chain where few others run
+// beside it: there chunks of more than 32 KiB go in two reads.  With head_dim 128
+// in 16 bits the other route runs the step beside the HCA pass, which hides it:
+// there the second read of K has to cost more than the step, from about 48 MiB
+// of K.  Measured, us a call, one read / two:
+//   bf16 D128: B8 H8 S16384 115 / 146, B1 H8 S32768 34.9 / 37.5, B1 H8 S16384
+//   24.9 / 24.5, S8192 21.7 / 18.5; HCA chunks of 512 KiB: 70.6 / 72.3;
+//   chunks of 32 KiB, 4 and 128 MiB of K: D64 f16 18.8 / 20.0, 55.7 / 77.2; f32
+//   D64 16.8 / 18.9, 53.8 / 74.7;
+//   64 KiB: D64 f16 of 32, 64, 128 items 22.4 / 20.6, 22.6 / 21.0, 22.9 / 24.0;
+//   D256 bf16 of 64 24.1 / 24.3; f32 D64 of 32 18.3 / 19.3;
+//   128 KiB: D64 f16 of 8, 128, 256, 512 31.1 / 22.6, 31.2 / 27.2, 32.5 / 32.2,
+//   38.1 / 47.4; D256 bf16 of 32, 128, 256 28.6 / 26.1, 28.9 / 27.8, 31.1 / 34.6;
+//   f32 D64 of 32, 64 21.5 / 20.3, 20.6 / 21.7;
+//   512 KiB: f32 D256 of 64 43.5 / 40.9, 1024 207.8 / 292.8.
+inline bool csa_hybrid_one_read(int64_t esz, int64_t head_dim, int64_t hca_chunk, int64_t items) {
+  const int64_t bytes = hca_chunk * head_dim * esz, KiB = 1024;
+  int64_t fewest = 1;
+  if (bytes > 128 * KiB)
+    fewest = 512;
+  else if (bytes > 64 * KiB)
+    fewest = esz == 4 ? 64 : head_dim == 64 ? 257 : 256;
+  else if (bytes > 32 * KiB && esz == 2 && head_dim == 64)
+    fewest = 128;
+  if (items < fewest) return false;
+  return esz == 4 || head_dim != 128 || items * bytes >= (int64_t{48} << 20);
+}
+
 }  // namespace csahca

@@ -25,6 +25,7 @@
 //                     columns over workgroups keeps each one to a single round
 //                     trip of ~C x 128 bytes even at batch 1.
 #include "csa_device.hpp"
+#include "dispatch.hpp"
 #include "hca_device.hpp"
 
 #include <algorithm>
@@ -276,33 +277,22 @@ size_t hca_means_offset(int64_t n_scores) {
 }
 
 // CSAHCA_HYBRID_ONE_READ=0 / 1 turns hybrid_chunk_kernel off / on wherever it
-// applies (read per call); unset (-1): the rule of hybrid_one_read.
+// applies (read per call); unset (-1): the rule of csa_hybrid_one_read.
 int env_one_read() {
   const char* s = std::getenv("CSAHCA_HYBRID_ONE_READ");
   return s ? (std::atoi(s) != 0 ? 1 : 0) : -1;
 }
 
 // Whether the hybrid op that builds its own summaries reads K once
-// (hybrid_chunk_kernel).  A wavefront walks a whole HCA chunk, so one of more
-// than 128 KiB needs many beside it.  With head_dim 128 in 16 bits the other
-// route runs the step beside the HCA pass, which hides it: there the second
-// read of K has to cost more than the step, from about 48 MiB of K.  Measured,
-// us a call, one read / two:
-//   bf16 D128: B8 H8 S16384 115 / 146, B1 H8 S32768 34.9 / 37.5, B1 H8 S16384
-//   24.9 / 24.5, S8192 21.7 / 18.5; HCA chunks of 2048: 70.6 / 72.3;
-//   D64 f16 B4 H8 S16384 35.0 / 46.2, B1 H4 S2048 16.4 / 17.4; f32 D128 B1 H8
-//   S16384 34.4 / 44.6, S2048 23.1 / 24.2; f32 D256 B1 H4 S4096 with 64
-//   wavefronts of 512 KiB 53.3 / 52.2.
+// (hybrid_chunk_kernel): whole CSA chunks of whole row groups, and the measured
+// rule (csa_hybrid_one_read).
 bool hybrid_one_read(int dtype, int64_t head_dim, int64_t csa_chunk, int64_t hca_chunk, int64_t items) {
   if (dtype == CSAHCA_F64 || (head_dim != 64 && head_dim != 128 && head_dim != 256)) return false;
   const int64_t esz = dtype == CSAHCA_F32 ? 4 : 2;
-  if (hca_chunk % csa_chunk != 0 || csa_chunk % (kHcaThreads * (16 / esz) / head_dim) != 0)
-    return false;  // whole CSA chunks of whole row groups
+  if (hca_chunk % csa_chunk != 0 || csa_chunk % (kHcaThreads * (16 / esz) / head_dim) != 0) return false;
   const int env = env_one_read();
   if (env >= 0) return env == 1;
-  const int64_t bytes = hca_chunk * head_dim * esz;
-  if (bytes > 128 * 1024 && items < 512) return false;
-  return esz == 4 || head_dim != 128 || items * bytes >= (int64_t{48} << 20);
+  return csa_hybrid_one_read(esz, head_dim, hca_chunk, items);
 }
 }  // namespace
 

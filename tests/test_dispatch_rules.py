@@ -13,6 +13,9 @@ extern "C" {
 int64_t split_tile(int64_t tile, int64_t total, int64_t bh, int64_t D, int64_t esz, int vec) {
   return csahca::csa_split_tile(tile, total, bh, D, esz, vec != 0);
 }
+int hybrid_one_read(int64_t esz, int64_t D, int64_t hca_chunk, int64_t items) {
+  return csahca::csa_hybrid_one_read(esz, D, hca_chunk, items);
+}
 int select_topk_regs(int64_t C, int64_t k) { return csahca::csa_select_topk_regs(C, k); }
 int step_topk_regs(int64_t C, int64_t k, int64_t bh, int fine) {
   return csahca::csa_step_topk_regs(C, k, bh, fine != 0);
@@ -32,6 +35,7 @@ def rules(tmp_path_factory):
     lib.split_tile.argtypes = [ctypes.c_int64] * 5 + [ctypes.c_int]
     lib.step_topk_regs.argtypes = [ctypes.c_int64] * 3 + [ctypes.c_int]
     lib.select_topk_regs.argtypes = [ctypes.c_int64] * 2
+    lib.hybrid_one_read.argtypes = [ctypes.c_int64] * 4
     return lib
 
 
@@ -115,3 +119,26 @@ def test_step_selection_registers_hold_every_key(rules):
 def test_selection_op_takes_registers_up_to_192_chunks(rules, C, k, want):
     """129-192 chunks went to the workgroup's top-k, 2-6% slower a call."""
     assert rules.select_topk_regs(C, k) == want
+
+
+@pytest.mark.parametrize("esz,D,hca_chunk,items,want", [
+    (2, 64, 256, 1, 1),         # 32 KiB an item
+    (2, 64, 512, 127, 0),       # 64 KiB: one read 7-9% slower
+    (2, 64, 512, 128, 1),
+    (2, 64, 1024, 256, 0),      # 128 KiB: 15-38% slower
+    (2, 64, 1024, 512, 1),
+    (2, 256, 128, 1, 1),
+    (2, 256, 256, 255, 0),      # 4-10% slower
+    (2, 256, 256, 256, 1),
+    (4, 64, 256, 1, 1),
+    (4, 64, 512, 63, 0),        # 6% slower
+    (4, 64, 512, 64, 1),
+    (4, 256, 256, 511, 0),      # more than 128 KiB
+    (4, 256, 256, 512, 1),
+    (2, 128, 256, 767, 0),      # 16-bit head_dim 128: from 48 MiB of K
+    (2, 128, 256, 768, 1),
+    (2, 128, 2048, 511, 0),
+    (4, 128, 64, 1, 1),
+])
+def test_hybrid_reads_k_once_where_wavefronts_are_many(rules, esz, D, hca_chunk, items, want):
+    assert rules.hybrid_one_read(esz, D, hca_chunk, items) == want
