@@ -4,9 +4,11 @@
 //   1. csa_summary_*   : fp32 mean of every chunk of K (the chunk summaries).
 //   2. csa_score_*     : score[c] = (q . summary[c]) / sqrt(D) in fp32, stored as
 //                        an order-preserving uint32 key.
-//   3. csa_topk_kernel : per (b,h) one wavefront loads the keys into LDS once and
-//                        selects the top-k (radix select + rank; score desc,
-//                        chunk id asc).
+//   3. csa_topk_kernel : per (b,h) the top-k of the keys (score desc, chunk id
+//                        asc): one wavefront from its registers up to 192 chunks
+//                        (csa_select_topk_regs), else four (block_topk for k <=
+//                        64, the first one's radix select for more), with the
+//                        keys in LDS where they fit and from memory where not.
 //   4. csa_attend_*    : split-KV sparse attention.  Work item = one wavefront
 //                        over `tile` consecutive selected-token slots of one
 //                        (b,h); K/V rows are fetched with 16-byte lane loads so

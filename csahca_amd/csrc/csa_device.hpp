@@ -309,7 +309,8 @@ __device__ bool wave_topk_regs(const uint32_t* keys, int C, int k, uint32_t* scr
 // aligned; lists: W * 65 words.  Contains barriers; the caller orders the last
 // reads of cand and lists.
 // Bound by its chain of LDS round trips and, from a few thousand keys, by the
-// reads: C / (64 W) a lane, twice.  (One wavefront's radix select, the only
+// reads: C / (64 W) a lane, twice, and a third time in lanes that hold a
+// candidate (keys in LDS, or in global memory where they do not fit).  (One wavefront's radix select, the only
 // path above 2048 keys before, reads every key 6 times with LDS atomics: B1 H8
 // D128 f32, 6295 chunks, top-14: 66.1 us a step, with this 23.2; B2 H8 D64 f32,
 // 3142 chunks, top-56: 43.8, 16.6.)

@@ -1588,7 +1588,7 @@ __global__ __launch_bounds__(NW * kWave) void dsv4_onepass_kernel(const int32_t*
 //     compiler ran the MFMAs and the conversions one after the other).
 // 64 heads of 512 fp32 sums and the bf16 query operand fill 256 of the 512
 // registers of a lane at one wavefront per SIMD; the tiles (two of 64 slots)
-// and P fill 146 KiB of LDS.  What bounds it: HBM at 256 queries (130 MB in
+// and P fill 143 KiB of LDS.  What bounds it: HBM at 256 queries (130 MB in
 // 39.5 us with 640 slots, 3.3 TB/s; the per-query kernel took 138.5 us), and
 // below that its serial chain, ~2.05 us a round (QK 0.7, softmax 0.3, PV 1.0)
 // and ~8 us around the rounds (query rows, first rows, output).

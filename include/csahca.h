@@ -81,7 +81,10 @@ int csahca_csa_decode_forward(const void* q, const void* k_cache, const void* v_
 
 /* Replaces csa_decode_forward_tiled_cuda (csrc/csa_attention.cu:387-452; pybind
  * op csa_decode_forward_tiled, bindings.cpp:66-77).  Same result; tile_size (> 0)
- * is the number of selected-token slots per split-KV work item. */
+ * is the least number of selected-token slots per split-KV work item: the
+ * library takes a multiple of it where longer items are faster (at most one
+ * batch of loads for short selections, 128 slots and more for long ones).
+ * The workspace is sized for tile_size itself. */
 int csahca_csa_decode_forward_tiled(const void* q, const void* k_cache, const void* v_cache,
                                     const void* chunk_indices, void* out, int dtype,
                                     int index_dtype, int64_t batch, int64_t heads,
@@ -89,7 +92,8 @@ int csahca_csa_decode_forward_tiled(const void* q, const void* k_cache, const vo
                                     int64_t chunk_size, int64_t tile_size, void* workspace,
                                     size_t workspace_bytes, void* stream);
 
-/* Split size the library picks for a CSA decode of this shape (>= 1). */
+/* The tile_size csahca_csa_decode_forward passes for a CSA decode of this shape
+ * (>= 1; like any tile_size, a lower bound). */
 int64_t csahca_csa_auto_tile_size(int64_t batch, int64_t heads, int64_t top_k,
                                   int64_t chunk_size);
 

@@ -75,7 +75,7 @@ def test_headline_decode_step():
     ref32 = oracle.csa_attend(case.q, case.k_cache, case.v_cache, want, 64, prob_dtype=oracle.F32)
     ref_torch_csa = oracle.csa_reference(case.q, case.k_cache, case.v_cache, chunk_size=64, top_k=8,
                                          selected_chunks=want, dtype=torch.bfloat16)
-    for tile in (8, 16, 64, native.csa_auto_tile_size(1, 8, 8, 64)):
+    for tile in (8, 16, 48, 64, 128, 512, native.csa_auto_tile_size(1, 8, 8, 64)):
         out = extension.csa_decode_forward_tiled(q, k, v, idx, 64, tile)
         assert_close(out, ref32, 2e-2, 1e-2, f"tile={tile}")
         assert_close(out, ref_torch_csa, 2e-2, 1e-2, f"vs torch-csa tile={tile}")
@@ -219,7 +219,7 @@ def test_deterministic_and_tile_invariant():
     b = extension.csa_decode_forward_tiled(q, k, v, idx, 64, 16)
     assert torch.equal(a, b)
     assert torch.equal(idx, extension.csa_select_topk(q, summ, 16))
-    outs = [extension.csa_decode_forward_tiled(q, k, v, idx, 64, t).float() for t in (1, 8, 64, 1024)]
+    outs = [extension.csa_decode_forward_tiled(q, k, v, idx, 64, t).float() for t in (1, 8, 48, 64, 128, 1024)]
     for o in outs[1:]:
         assert torch.allclose(o, outs[0], atol=1e-2, rtol=1e-2)
 

@@ -92,22 +92,52 @@ def test_wide_kernel_matches_oracle(heads, top_k, extra_top_k, page, extra_page,
     assert_close(gpu_out(c, sink=False), oracle_out(c, sink=False))
 
 
-@pytest.mark.parametrize("jump", [0.5, 40.0, 4000.0])
-def test_wide_kernel_scores_that_outgrow_the_first_round(jump):
-    """Probabilities are formed against the first round's maximum; later scores
-    that exceed it by up to 2^64 (jump 40: some tens of nats) are kept as they
-    are, larger ones (jump 4000) take the second walk.  Against the oracle and
-    against the other kernels, whose maximum moves."""
+def excess_bits(c, rows):
+    """Per query, how far (log2) the best later score of any head exceeds that
+    head's maximum over the first 64 slots."""
+    x = torch.einsum("qhd,sd->qhs", c.q.double(), rows.to(torch.bfloat16).double()) * SCALE / math.log(2)
+    return (x[..., 64:].amax(-1) - x[..., :64].amax(-1)).amax(-1)
+
+
+@pytest.mark.parametrize("jump,low,high", [
+    (0.5, -math.inf, 7), (2.0, 9, 60), (4.0, 18, 60), (8.0, 36, 62), (40.0, 80, math.inf), (4000.0, 80, math.inf),
+])
+def test_wide_kernel_scores_that_outgrow_the_first_round(jump, low, high):
+    """Probabilities are formed against the first round's maximum: later scores
+    that exceed it by up to 2^8 and by up to 2^64 are kept as they are, larger
+    ones take the second walk.  `low` and `high` bound the excess of every
+    query, with room for the cache's rounding of the rows, so that each stays
+    in its regime.  Against the oracle."""
     c = make_dsv4_case(compress_ratio=0, num_queries=5, heads=64, num_tokens=512, top_k=200, page_size=64,
                        full_lengths=True, seed=3, pack=False, device="cpu")
     c.token_indices = torch.arange(200, dtype=torch.int32).repeat(5, 1)
     rows = c.k_tokens.float()
     rows[:64] *= 0.01
     rows[130:] *= jump
+    excess = excess_bits(c, rows[:200])
+    assert low < excess.min() and excess.max() < high, excess
     c.cache = pack_dsv4_cache(rows.to(torch.bfloat16), page_size=64)
     ref = oracle_out(c)
     # the outputs are of the rows' own magnitude: the bar relative to it
     assert_close(gpu_out(c) / max(jump, 1.0), ref / max(jump, 1.0))
+
+
+def test_wide_kernel_accumulators_that_overflow_the_first_walk():
+    """A late score 40 bits above the first round's maximum over rows of 1e28: the
+    accumulators overflow against that maximum, not against the true one, so
+    the list is walked again."""
+    c = make_dsv4_case(compress_ratio=0, num_queries=3, heads=64, num_tokens=200, top_k=200, page_size=64,
+                       full_lengths=True, seed=5, pack=False, device="cpu")
+    c.token_indices = torch.arange(200, dtype=torch.int32).repeat(3, 1)
+    c.q[:, :, 500], c.q[:, :, 510] = 8.0, 0.0
+    c.k_tokens[:, 500], c.k_tokens[:, 510] = 0.0, 1e28
+    c.k_tokens[150, 500] = 40 * math.log(2) * math.sqrt(512) / 8.0
+    excess = excess_bits(c, c.k_tokens)
+    assert 28 < excess.min() and excess.max() < 60, excess
+    c.cache = pack_dsv4_cache(c.k_tokens, page_size=64)
+    ref = oracle_out(c)
+    assert np.isfinite(ref).all() and abs(ref[..., 510]).min() > 5e27
+    assert_close(gpu_out(c), ref)
 
 
 def test_wide_kernel_scale_byte_255_poisons_its_query_only():
