@@ -336,7 +336,7 @@ def csa_bench(args, B=1, H=8, S=32768, D=128, chunk=64, top_k=8, copies=None, se
     return res
 
 
-STEP_KERNEL_SOURCES = ("csa_step.hip", "csa_device.hpp", "common.hpp", "hca_device.hpp")
+STEP_KERNEL_SOURCES = ("csa_step.hip", "csa_device.hpp", "common.hpp", "hca_device.hpp", "dispatch.hpp")
 
 
 def step_kernel_sources_sha256() -> str:

@@ -1,6 +1,7 @@
 """The rules on sizes that choose a launch (csahca_amd/csrc/dispatch.hpp), built
 alone with the host compiler."""
 import ctypes
+import re
 import subprocess
 from pathlib import Path
 
@@ -142,3 +143,17 @@ def test_selection_op_takes_registers_up_to_192_chunks(rules, C, k, want):
 ])
 def test_hybrid_reads_k_once_where_wavefronts_are_many(rules, esz, D, hca_chunk, items, want):
     assert rules.hybrid_one_read(esz, D, hca_chunk, items) == want
+
+
+def test_the_step_kernels_traffic_record_covers_every_source():
+    """bench.py reports profiles/traffic.json only for the sources it names; the
+    rules' header picks the step's instantiation and was not among them."""
+    bench = (CSRC.parents[1] / "bench.py").read_text()
+    named = set(re.findall(r'"([^"]+)"', re.search(r"STEP_KERNEL_SOURCES = \(([^)]*)\)", bench).group(1)))
+    seen, todo = set(), ["csa_step.hip"]
+    while todo:
+        name = todo.pop()
+        if name not in seen and (CSRC / name).exists():
+            seen.add(name)
+            todo += re.findall(r'#include "([^"]+)"', (CSRC / name).read_text())
+    assert named == seen
