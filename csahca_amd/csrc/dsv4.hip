@@ -507,34 +507,7 @@ __device__ __forceinline__ uint4 dequant8_bf16(uint2 w, uint32_t sbyte) {
                       bf16x2_bits(__builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w.y, s, false)),
                       bf16x2_bits(__builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w.y, s, true)));
   }
-  const float s = ue8m0_to_f32(sbyte);
-  uint32_t o[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const uint32_t word = i < 2 ? w.x : w.y;
-    const uint32_t b0 = (word >> (16 * (i & 1))) & 0xffu;
-    const uint32_t b1 = (word >> (16 * (i & 1) + 8)) & 0xffu;
-    o[i] = static_cast<uint32_t>(float_to_bf16_bits(e4m3_to_f32(b0) * s)) |
-           (static_cast<uint32_t>(float_to_bf16_bits(e4m3_to_f32(b1) * s)) << 16);
-  }
-  return make_uint4(o[0], o[1], o[2], o[3]);
-}
-
-// Eight codes by way of fp32 (exact e4m3 values, an fp32 product, round to
-// nearest even): the software decode's results for every scale byte, in 16
-// instructions.
-__device__ __forceinline__ uint4 dequant8_bf16_f32(uint2 w, uint32_t sbyte) {
-  typedef float f32x2_v __attribute__((ext_vector_type(2)));
-  const float s = ue8m0_to_f32(sbyte);
-  uint32_t o[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int word = static_cast<int>(i < 2 ? w.x : w.y);
-    const f32x2_v v = (i & 1) ? __builtin_amdgcn_cvt_pk_f32_fp8(word, true) : __builtin_amdgcn_cvt_pk_f32_fp8(word, false);
-    const bf16x2_t b = {static_cast<__bf16>(v[0] * s), static_cast<__bf16>(v[1] * s)};
-    o[i] = bf16x2_bits(b);
-  }
-  return make_uint4(o[0], o[1], o[2], o[3]);
+  return dequant8_bf16_sw(w, sbyte);
 }
 
 // How a (query, head group, split) workgroup finishes.
@@ -1588,10 +1561,15 @@ __global__ __launch_bounds__(NW * kWave) void dsv4_onepass_kernel(const int32_t*
 //     compiler ran the MFMAs and the conversions one after the other).
 // 64 heads of 512 fp32 sums and the bf16 query operand fill 256 of the 512
 // registers of a lane at one wavefront per SIMD; the tiles (two of 64 slots)
-// and P fill 143 KiB of LDS.  What bounds it: HBM at 256 queries (130 MB in
-// 39.5 us with 640 slots, 3.3 TB/s; the per-query kernel took 138.5 us), and
-// below that its serial chain, ~2.05 us a round (QK 0.7, softmax 0.3, PV 1.0)
-// and ~8 us around the rounds (query rows, first rows, output).
+// and P fill 143 KiB of LDS.  What bounds it: the serial chain of that one
+// wavefront, ~2.05 us a round (QK 0.7, softmax 0.3, PV 1.0) and ~8 us around the
+// rounds (query rows, first rows, output): 640 slots take 29.8 us at 32 queries
+// and 30.7 at 64, on a quarter of the CUs.  At 256 queries the wavefronts wait
+// 6-8 us longer for their rows (37-40 us; the per-query kernel 135-138): issuing
+// 48% of their cycles, waiting for memory or LDS 32%, for an issue slot 20%, MFMA
+// busy 19%; 148 MB in 38.9 us is 3.8 TB/s, where a read stream reaches 5.8.  It
+// fetches 693 bytes a slot for the 584 of a row and its scales: a row is 4.5
+// lines of 128 bytes, the scales lie in a line of their own.
 // MFMA layouts (32x32x16): A lane l elem j = A[l%32][8(l/32)+j], B lane l elem
 // j = B[8(l/32)+j][l%32], C lane l elem i = C[8(i/4)+4(l/32)+i%4][l%32].
 // ---------------------------------------------------------------------------
@@ -1796,7 +1774,7 @@ __global__ __launch_bounds__(kWideWaves * kWave, 1) void dsv4_wide_kernel(const 
     const uint2 w = h ? make_uint2(c.z, c.w) : make_uint2(c.x, c.y);
     uint4 v;
     if constexpr (decltype(general)::value)
-      v = dequant8_bf16_f32(w, sbyte);
+      v = dequant8_bf16_sw(w, sbyte);
     else
       v = dequant8_bf16_hw(w, sbyte);
     uint16_t* dst = trow + 16 * (c8 + 8 * j) + 8 * h;
