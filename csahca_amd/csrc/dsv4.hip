@@ -2309,14 +2309,15 @@ bool use_onepass(int64_t total_slots) {
 //     / 33.3 / 46.1 us a call against 38.4 / 46.8 / 69.5 / 106.0).
 //   * Fewer, down to a quarter: one wave there, and a round of 64 slots takes the
 //     wide kernel 2.05 us against 2.9, so it is behind up to the length where
-//     that makes up for its 8 us around the rounds and for a last round that
-//     is not full (its masks: 1.2 us).  nq 32 x H 64, 320 / 352 / 384 / 448 /
-//     512 slots: 20.2 / 23.4 / 22.1 / 24.4 / 26.3 against 19.4 / 21.6 / 22.1 /
-//     25.3 / 28.1; nq 40 (160 pairs, two dim parts no longer fit): 20.3 / 23.5 /
-//     22.3 / 24.5 / 26.7 against 20.9 / 23.2 / 23.9 / 26.8 / 29.7; nq 64 20.5 /
-//     23.9 / 22.6 / 24.8 / 27.0 against 21.3 / 23.9 / 24.5 / 27.8 / 30.8; the
-//     same line at H 24, 32, 80 and 128.  Below half, nq 24 x H 64, 384 / 448 /
-//     512: 22.2 / 24.3 / 26.3 against 22.0 / 24.9 / 27.9.
+//     that makes up for its 8 us around the rounds and for rounds that are not
+//     full (their masks: 1.2 us), which lists shorter than their slots end in.
+//     Ratio of the times, full lists / lists of half to all of their slots, at
+//     384, 448, 480, 512, 576, 640 slots: more than half a pair per CU (two dim
+//     parts no longer fit there) .95 / 1.04, .92 / 1.01, .95 / .99, .90 / .98, .88 /
+//     .95, .86 / .93; 80 to 128 pairs 1.02 / 1.13, .98 / 1.08, 1.02 / 1.06, .95 /
+//     1.05, .93 / 1.02, .92 / 1.00; 64 pairs 1.04 / 1.17, 1.01 / 1.12, 1.05 / 1.06,
+//     .98 / 1.07, .96 / 1.06, .94 / 1.03 (704: .92 / 1.01); 320 slots .99 / 1.09 at
+//     best.  The same at H 24, 32, 48, 64 and 128.  The lines: 448, 576, 640.
 //   * Fewer still take the split kernel.
 // With 16 heads or fewer three quarters of its MFMA work would be padding (nq
 // 256, 192 slots 15.7 against 17.6).
@@ -2337,8 +2338,7 @@ bool use_wide(int64_t nq, int64_t heads, int64_t total_slots) {
   const int64_t pairs = nq * ceil_div(heads, kQHeads);
   if (heads <= kQHeads || ncu <= 0 || total_slots <= kOpMaxSlots || 4 * pairs < ncu) return false;
   if (pairs <= ncu) {
-    const bool whole = total_slots % kWideSlots == 0;
-    const int64_t line = 8 * pairs >= 5 * ncu && whole ? 320 : 2 * pairs >= ncu ? 384 : 512;
+    const int64_t line = 2 * pairs > ncu ? 448 : 16 * pairs >= 5 * ncu ? 576 : 640;
     if (total_slots < line) return false;
   }
   const char* f = env_switch("CSAHCA_DSV4_QUERY");

@@ -289,17 +289,18 @@ def kernels_of(call):
 @pytest.mark.parametrize("nq,heads,slots,wide", [
     (72, 64, 257, True),    # more (query, 16 heads) pairs than CUs
     (72, 64, 256, False),   # the longest list of the one-pass kernel
-    (64, 64, 304, False),   # 256 pairs
-    (64, 64, 320, True),    # whole rounds
-    (64, 64, 352, False),
-    (64, 64, 384, True),
-    (32, 64, 320, False),   # 128 pairs
-    (32, 64, 383, False),
-    (32, 64, 384, True),
-    (31, 64, 384, False),   # 124 pairs
-    (31, 64, 512, True),
-    (16, 64, 512, True),    # 64 pairs
-    (15, 64, 512, False),
+    (64, 64, 384, False),   # 256 pairs
+    (64, 64, 447, False),
+    (64, 64, 448, True),
+    (33, 64, 448, True),    # 132 pairs
+    (32, 64, 448, False),   # 128 pairs
+    (32, 64, 575, False),
+    (32, 64, 576, True),
+    (20, 64, 576, True),    # 80 pairs
+    (19, 64, 576, False),
+    (16, 64, 639, False),   # 64 pairs
+    (16, 64, 640, True),
+    (15, 64, 640, False),
     (1, 256, 384, False),   # 16 pairs, in a grid of 128
     (1, 256, 640, False),
     (4, 256, 640, True),    # 64 pairs
