@@ -7,13 +7,12 @@
 
 namespace csahca {
 
-// Slots per wavefront of the split-KV attention: the caller's tile, or a
-// multiple of it where more slots per wavefront are better.  A tile is a hint
-// for the split, and the partials of several of the caller's tiles are one
-// partial of their union, so the workspace the caller sized for its own tile
-// holds them.  `vec`: the vectorised kernel runs (esz: bytes per element).
+// Slots per wavefront of the split-KV attention: the caller's tile, or more
+// where that is better.  A tile is a hint for the split, and larger tiles are
+// fewer partials, so the workspace the caller sized for its own tile holds
+// them.  `vec`: the vectorised kernel runs (esz: bytes per element).
 //
-// The smallest multiple that, for the vectorised kernel,
+// The least number of whole load batches that, for the vectorised kernel,
 //   * fills one batch of row loads (16 slots at 16-bit head_dim 128, 32 at 64;
 //     a smaller tile re-reads its last row);
 //   * leaves a head at most 64 tiles, the one-round-trip merge, as long as that
@@ -23,14 +22,17 @@ namespace csahca {
 // Measured (graph period, us, tile 8 as called / split chosen): B1 H8 D128
 // top-8 5.31 / 5.06, top-32 49.3 / 7.3; B8 top-16 16.4 / 10.3, top-32 60.6 /
 // 15.3; B32 top-32 104.7 / 56.7; B4 H12 D64 f16 480 slots 7.3 / 6.4; f32 D256
-// 512 slots 9.4 (kept at 8).
+// 512 slots 9.4 (kept at 8).  Multiples of the caller's tile would pass the line
+// by up to a tile, a serial chain twice as long: f32 D128 H12 4352 slots, tile
+// 64, with tiles of 64 / 72 / 128 20.0 / 17.0 / 24.4; f32 D64 H8 6000, tile 80, of
+// 80 / 96 / 160 14.2 / 11.6 / 15.5.
 //
 // Generic kernel: its wavefronts take 4 slots per round trip, 0.23 us a slot at
 // D 40 to 0.39 at D 320 f32, so long tiles are a long serial chain, and the
 // merge of more than 64 partials is the cheaper side until the rows themselves
 // take that long to stream: the same line, with 12800 wavefronts for rows below
-// 1 KiB, but no multiple above 16 slots, 32 from 100 MiB of rows, any from 200
-// MiB of rows of at least 384 bytes.  Measured, us, with tiles of 8 / 16 / 32 /
+// 1 KiB, but at most 16 slots, 32 from 100 MiB of rows, any number from 200 MiB
+// of rows of at least 384 bytes.  Measured, us, with tiles of 8 / 16 / 32 /
 // 64 (and by the vectorised kernel's line): D40 bf16 B1 H8 3200 slots 12.7 /
 // 11.6 / 13.1 / 19.4 (16.7); D96 bf16 B1 1600 slots 9.6 / 10.1 / 13.2 / 21.2
 // (12.1), B4 6400 35.7 / 32.3 / 32.8 / 38.9 (41.4), B32 1600 53.4 / 50.1 / 49.3
@@ -43,14 +45,11 @@ inline int64_t csa_split_tile(int64_t tile, int64_t total, int64_t bh, int64_t D
   const int64_t batch = vec ? 4 * (kLanes / (D * esz / 16)) : 4;
   const int64_t waves = vec || D * esz >= 1024 ? 8192 : 12800;
   int64_t want = std::max({batch, std::min<int64_t>(ceil_of(total, kOneTripTiles), 128), ceil_of(total * bh, waves)});
-  int64_t most = INT64_MAX;
   if (!vec) {
     const double mib = 2.0 * static_cast<double>(total) * static_cast<double>(bh * D * esz) / (1 << 20);
-    if (mib < 200.0 || D * esz < 384) most = mib < 100.0 ? 16 : 32;
-    want = std::min(want, most);
+    if (mib < 200.0 || D * esz < 384) want = std::min<int64_t>(want, mib < 100.0 ? 16 : 32);
   }
-  int64_t t = tile;
-  if (tile < want) t = std::min(ceil_of(want, tile), most / tile) * tile;
+  const int64_t t = std::max(tile, ceil_of(want, batch) * batch);
   return std::min<int64_t>(t, std::max<int64_t>(total, 1));
 }
 

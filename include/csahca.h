@@ -82,7 +82,7 @@ int csahca_csa_decode_forward(const void* q, const void* k_cache, const void* v_
 /* Replaces csa_decode_forward_tiled_cuda (csrc/csa_attention.cu:387-452; pybind
  * op csa_decode_forward_tiled, bindings.cpp:66-77).  Same result; tile_size (> 0)
  * is the least number of selected-token slots per split-KV work item: the
- * library takes a multiple of it where longer items are faster (at most one
+ * library takes more where longer items are faster (at most one
  * batch of loads for short selections, 128 slots and more for long ones).
  * The workspace is sized for tile_size itself. */
 int csahca_csa_decode_forward_tiled(const void* q, const void* k_cache, const void* v_cache,

@@ -51,9 +51,9 @@ def rules(tmp_path_factory):
     (4, 400, 32, 96, 2, 8),
     (4, 200, 8, 96, 2, 4),
     (1, 64, 1, 96, 2, 4),
-    (3, 64, 1, 96, 2, 6),
-    (5, 3200, 8, 96, 2, 15),
-    (12, 3200, 8, 96, 2, 12),
+    (3, 64, 1, 96, 2, 4),
+    (5, 3200, 8, 96, 2, 16),
+    (12, 3200, 8, 96, 2, 16),
     (8, 3200, 256, 96, 2, 32),    # 300 MiB of rows of 192 bytes
     (16, 800, 256, 192, 2, 16),
     (4, 256, 256, 192, 2, 8),
@@ -72,7 +72,11 @@ def test_generic_split_keeps_its_chain_short(rules, tile, total, bh, D, esz, wan
     (8, 512, 16, 256, 4, 8),
     (8, 2048, 8, 128, 2, 32),     # 64 tiles a head
     (8, 1024, 64, 128, 2, 16),
-    (5, 192, 6, 128, 2, 20),
+    (5, 192, 6, 128, 2, 16),
+    (64, 4352, 12, 128, 4, 72),   # a tile just below the line: twice it was 1.22 times as slow
+    (80, 6000, 8, 64, 4, 96),     # 1.09
+    (72, 4352, 12, 128, 4, 72),
+    (200, 4352, 12, 128, 4, 200),
     (1, 16384, 1, 128, 2, 128),
     (8, 2048, 256, 128, 2, 64),   # 8192 wavefronts
 ])

@@ -17,13 +17,15 @@ DEV = "cuda"
     (1, 1, 8192, 128, 64, 128, 8, torch.bfloat16),     # 8192 slots: 64 tiles of 128, the last one-round-trip merge
     (1, 2, 12928, 128, 64, 202, 8, torch.bfloat16),    # 101 tiles
     (1, 1, 8256, 64, 64, 129, 1, torch.float16),       # 65 tiles: one past the one-round-trip merge
-    (1, 1, 132000, 64, 1000, 132, 7, torch.float16),   # 997 tiles of 133 slots
+    (1, 1, 132000, 64, 1000, 132, 7, torch.float16),   # 1032 tiles: two passes of weights, 8 in the second
+    (1, 1, 132000, 64, 1000, 132, 133, torch.float16), # 993 tiles of 133 slots, no whole load batches
     (1, 1, 140000, 64, 1000, 140, 8, torch.bfloat16),  # 1094 tiles: two passes of weights
     (2, 1, 9000, 96, 50, 180, 8, torch.bfloat16),      # generic kernel, 563 tiles; columns that are no multiple of 32
-    (1, 2, 9216, 256, 48, 190, 3, torch.float32),      # 72 tiles of 129 slots
+    (1, 2, 9216, 256, 48, 190, 3, torch.float32),      # 72 tiles of 128 slots
     (1, 1, 9216, 100, 64, 144, 8, torch.float64),      # generic kernel, 576 tiles, 100 columns
-    (3, 2, 640, 128, 64, 3, 5, torch.bfloat16),        # 192 slots: tiles of 20 for the asked 5
-    (1, 1, 64, 64, 16, 1, 3, torch.float16),           # 16 slots in one tile of at most 33
+    (1, 3, 4352, 128, 64, 68, 64, torch.float32),      # 61 tiles of 72 slots for the asked 64
+    (3, 2, 640, 128, 64, 3, 5, torch.bfloat16),        # 192 slots: tiles of 16 for the asked 5
+    (1, 1, 64, 64, 16, 1, 3, torch.float16),           # 16 slots in one tile of at most 32
 ])
 def test_split_matches_oracle(B, H, S, D, chunk, k, tile, dtype):
     g = torch.Generator().manual_seed(S + D + k)
