@@ -53,28 +53,39 @@ inline int64_t csa_split_tile(int64_t tile, int64_t total, int64_t bh, int64_t D
   return std::min<int64_t>(t, std::max<int64_t>(total, 1));
 }
 
+// The largest selection that the register path takes of C <= 2048 chunks (up to
+// 16 heads: few_heads).  It fails where more than 64 keys reach its threshold,
+// the k-th largest of the 64 lanes' maxima: never for k + C <= 128 distinct keys
+// (C - 64 lanes hold a second one), and of many independent keys 64 ln(64 / (64
+// - k)) reach it (44 for k = 32, 53 for 36, 63 for 40), fewer of few per lane.
+// The radix select behind it costs 6-20 us, and one head of the call that takes
+// it costs the call that.  So the line is where a call of all its heads still
+// rarely fails.  Simulated, failures a head: 96 chunks k = 43, 45 1e-4, 3e-3;
+// 128 k = 41, 43 5e-5, 2e-3; 144 k = 39, 41 2e-4, 2e-3; 192 k = 37, 39 5e-5, 1e-3;
+// 256 k = 36, 38, 40 9e-5, 2.6e-3, 2.7e-2; 512 k = 34, 36, 38 5e-5, 2.9e-3,
+// 2.6e-2; 2048 k = 34, 36, 38 1.1e-3, 1.3e-2, 7.9e-2.  Measured, registers (not
+// failing) against block_topk, us a step, B1 H8 D128 chunk 16: top-33 of 256,
+// 512, 1024, 2048: 9.4 / 10.1, 9.5 / 10.5, 11.6 / 11.7, 12.9 / 13.5; top-36 of 256,
+// 512: 9.4 / 10.1, 9.6 / 10.5; top-40 of 64, 128: 9.3 / 10.0, 9.3 / 9.8, and
+// failing, of 384: 17.6 / 10.5; top-64 of 64, 128, 512, 2048: 9.6 / 10.2, 18.3 /
+// 10.7, 21.4 / 11.5, 36.2 / 13.7; 48 heads of 64, top-37 of 132 12.9 / 13.9; 16
+// heads of 256, the selection op, top-50 of 65 6.3 / 6.7.
+inline int64_t csa_topk_regs_most(int64_t C, bool few_heads) {
+  if (C <= 64) return 64;
+  if (C <= 84) return 128 - C;
+  const int64_t most = C <= 96 ? 43 : C <= 128 ? 41 : C <= 144 ? 39 : C <= 192 ? 37 : C <= 256 ? 36 : C <= 512 ? 34 : 32;
+  return most + (few_heads ? 2 : 0);
+}
+
 // Register-path size for the fused step's selection of k of C chunks: keys per
 // lane M (C <= 64 * M), or 0 for block_topk (k <= 64) or the radix select.
 // Kernels take M as a template parameter so each instantiation carries exactly
-// one of them.  The register path fails where more than 64 keys reach its
-// threshold, which of independent keys 64 ln(64 / (64 - k)) do (44 for k = 32,
-// 53 for 36, 63 for 40), fewer of few per lane; the radix select behind it costs
-// 6-20 us, and one head of the call that takes it costs the call that.  So the
-// line for more than 128 chunks is where a call of all its heads still rarely
-// fails.  Simulated, failures a head at k = 34 / 36 / 38 / 40: 256 chunks <1e-5 /
-// 9e-5 / 2.6e-3 / 2.7e-2, 512 chunks 5e-5 / 2.9e-3 / 2.6e-2 / 0.13, 2048 chunks
-// 1.1e-3 / 1.3e-2 / 7.9e-2 / 0.27.  Measured, B1 H8 D128 chunk 16, registers
-// (not failing) against block_topk, us a step: top-33 of 256, 512, 1024, 2048:
-// 9.4 / 10.1, 9.5 / 10.5, 11.6 / 11.7, 12.9 / 13.5; top-36 of 256, 512: 9.4 / 10.1,
-// 9.6 / 10.5; top-40 of 64, 128: 9.3 / 10.0, 9.3 / 9.8, and failing, of 384: 17.6 /
-// 10.5; top-64 of 64, 128, 512, 2048: 9.6 / 10.2, 18.3 / 10.7, 21.4 / 11.5, 36.2 /
-// 13.7.
+// one of them.
 // The fewest keys per lane that hold C: `fine` where the kernels with 2 and 16
 // exist (head_dim 128 in 16 bits; bf16 us a step, top-8: 128 chunks with 8 and
 // with 2 7.92 / 7.59, 1024 with 32 and with 16 10.0 / 9.15).
 inline int csa_step_topk_regs(int64_t C, int64_t k, int64_t bh, bool fine) {
-  const int64_t most = C <= 64 ? 64 : C <= 128 ? 40 : (C <= 256 ? 36 : C <= 512 ? 34 : 32) + (bh <= 16 ? 2 : 0);
-  if (k > most || C > 2048) return 0;
+  if (C > 2048 || k > csa_topk_regs_most(C, bh <= 16)) return 0;
   if (fine && C <= 128) return 2;
   if (C <= 512) return 8;
   return fine && C <= 1024 ? 16 : 32;
@@ -86,9 +97,8 @@ inline int csa_step_topk_regs(int64_t C, int64_t k, int64_t bh, bool fine) {
 // 128: 5.2 / 5.4, 11.7 / 5.3; top-8 of 129, 160, 192: 4.94 / 5.32, 5.18 / 5.30,
 // 5.11 / 5.27; top-36 of 129, 192: 5.32 / 5.76, 5.56 / 5.72; top-16 level.
 inline int csa_select_topk_regs(int64_t C, int64_t k) {
-  if (C <= 64) return k <= 64 ? 2 : 0;
-  if (C <= 128) return k <= 40 ? 2 : 0;
-  return C <= 192 && k <= 36 ? 4 : 0;
+  if (C > 192 || k > csa_topk_regs_most(C, false)) return 0;
+  return C <= 128 ? 2 : 4;
 }
 
 // Whether the hybrid op reads K once for the summaries and the HCA chunk pass

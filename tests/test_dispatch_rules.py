@@ -5,6 +5,7 @@ import re
 import subprocess
 from pathlib import Path
 
+import numpy as np
 import pytest
 
 CSRC = Path(__file__).resolve().parents[1] / "csahca_amd" / "csrc"
@@ -98,17 +99,36 @@ def test_split_fits_the_callers_workspace(rules, vec):
 
 
 @pytest.mark.parametrize("C,k,bh,fine,want", [
-    (1, 1, 1, 1, 2), (64, 64, 8, 1, 2), (64, 64, 8, 0, 8), (128, 40, 256, 1, 2), (128, 41, 8, 1, 0),
-    (129, 36, 256, 1, 8), (129, 37, 17, 1, 0), (256, 38, 16, 1, 8), (256, 39, 8, 1, 0),
+    (1, 1, 1, 1, 2), (64, 64, 8, 1, 2), (64, 64, 8, 0, 8), (64, 65, 1, 1, 0),
+    (65, 63, 256, 1, 2), (65, 64, 8, 1, 0), (84, 44, 256, 1, 2), (84, 45, 8, 1, 0),
+    (96, 43, 256, 0, 8), (96, 45, 16, 1, 2), (96, 44, 17, 1, 0), (128, 41, 256, 1, 2), (128, 44, 8, 1, 0),
+    (132, 37, 48, 0, 8), (144, 39, 256, 1, 8), (144, 42, 8, 1, 0), (192, 37, 17, 1, 8), (192, 38, 17, 1, 0),
+    (193, 36, 256, 1, 8), (193, 37, 17, 1, 0), (256, 38, 16, 1, 8), (256, 39, 8, 1, 0),
     (257, 34, 256, 1, 8), (512, 35, 17, 1, 0), (512, 36, 16, 0, 8), (512, 37, 8, 1, 0),
     (513, 32, 256, 1, 16), (513, 32, 256, 0, 32), (1024, 33, 17, 1, 0), (1024, 34, 16, 1, 16), (1024, 35, 8, 1, 0),
-    (1025, 32, 256, 1, 32), (2048, 34, 8, 1, 32), (2048, 35, 8, 1, 0), (2049, 1, 1, 1, 0),
-    (64, 65, 1, 1, 0), (512, 100, 1, 1, 0),
+    (1025, 32, 256, 1, 32), (2048, 34, 8, 1, 32), (2048, 35, 8, 1, 0), (2049, 1, 1, 1, 0), (512, 100, 1, 1, 0),
 ])
 def test_step_selection_takes_registers_where_they_rarely_fail(rules, C, k, bh, fine, want):
-    """33-38 of more than 128 chunks went to all wavefronts, 5-10% slower a step
-    than one wavefront's registers."""
+    """33-38 of more than 128 chunks, and 41-63 of up to 128 that cannot or hardly
+    fail, went to all wavefronts, 5-10% slower a step than one wavefront's
+    registers."""
     assert rules.step_topk_regs(C, k, bh, fine) == want
+
+
+def test_step_selection_registers_cannot_fail_up_to_84_chunks(rules):
+    """Lane L of 64 holds keys L, L + 64 (rotated); the threshold is the k-th
+    largest lane maximum; 64 candidates fit."""
+    rng = np.random.default_rng(0)
+    for C in range(65, 85):
+        k = max(k for k in range(1, 65) if rules.step_topk_regs(C, k, 256, 1))
+        assert k == 128 - C
+        keys = np.full((200, 128), -1)
+        keys[:, :C] = rng.random((200, C)).argsort(-1)
+        keys[:20, :C] = np.arange(C)         # the second row holds the largest
+        keys[20:40, :C] = np.arange(C)[::-1]
+        lanes = keys.reshape(200, 2, 64).max(1)
+        t = np.sort(lanes, -1)[:, 64 - k]
+        assert (keys >= t[:, None]).sum(-1).max() <= 64
 
 
 def test_step_selection_registers_hold_every_key(rules):
@@ -119,10 +139,12 @@ def test_step_selection_registers_hold_every_key(rules):
 
 
 @pytest.mark.parametrize("C,k,want", [
-    (1, 1, 2), (64, 64, 2), (64, 65, 0), (128, 40, 2), (128, 41, 0), (129, 1, 4), (192, 36, 4), (192, 37, 0), (193, 1, 0),
+    (1, 1, 2), (64, 64, 2), (64, 65, 0), (65, 63, 2), (65, 64, 0), (84, 44, 2), (84, 45, 0), (96, 43, 2), (96, 44, 0),
+    (128, 41, 2), (128, 42, 0), (129, 1, 4), (129, 39, 4), (192, 37, 4), (192, 38, 0), (193, 1, 0),
 ])
 def test_selection_op_takes_registers_up_to_192_chunks(rules, C, k, want):
-    """129-192 chunks went to the workgroup's top-k, 2-6% slower a call."""
+    """129-192 chunks, and 41-63 of 65-84, went to the workgroup's top-k, 2-7%
+    slower a call."""
     assert rules.select_topk_regs(C, k) == want
 
 
