@@ -104,31 +104,42 @@ inline int csa_select_topk_regs(int64_t C, int64_t k) {
 // Whether the hybrid op reads K once for the summaries and the HCA chunk pass
 // (`items` HCA chunks of hca_chunk rows over all heads).  A wavefront walks a
 // whole HCA chunk of one tensor, and is the longer chain where few others run
-// beside it: there chunks of more than 32 KiB go in two reads.  With head_dim 128
-// in 16 bits the other route runs the step beside the HCA pass, which hides it:
-// there the second read of K has to cost more than the step, from about 48 MiB
-// of K.  Measured, us a call, one read / two:
-//   bf16 D128: B8 H8 S16384 115 / 146, B1 H8 S32768 34.9 / 37.5, B1 H8 S16384
-//   24.9 / 24.5, S8192 21.7 / 18.5; HCA chunks of 512 KiB: 70.6 / 72.3;
-//   chunks of 32 KiB, 4 and 128 MiB of K: D64 f16 18.8 / 20.0, 55.7 / 77.2; f32
-//   D64 16.8 / 18.9, 53.8 / 74.7;
-//   64 KiB: D64 f16 of 32, 64, 128 items 22.4 / 20.6, 22.6 / 21.0, 22.9 / 24.0;
-//   D256 bf16 of 64 24.1 / 24.3; f32 D64 of 32 18.3 / 19.3;
-//   128 KiB: D64 f16 of 8, 128, 256, 512 31.1 / 22.6, 31.2 / 27.2, 32.5 / 32.2,
-//   38.1 / 47.4; D256 bf16 of 32, 128, 256 28.6 / 26.1, 28.9 / 27.8, 31.1 / 34.6;
-//   f32 D64 of 32, 64 21.5 / 20.3, 20.6 / 21.7;
-//   512 KiB: f32 D256 of 64 43.5 / 40.9, 1024 207.8 / 292.8.
-inline bool csa_hybrid_one_read(int64_t esz, int64_t head_dim, int64_t hca_chunk, int64_t items) {
-  const int64_t bytes = hca_chunk * head_dim * esz, KiB = 1024;
+// beside it, the more so the fewer row groups (4096 bytes of K) lie in a CSA
+// chunk, whose end it stops to reduce: there long chunks go in two reads.  With
+// head_dim 128 in 16 bits the other route runs the step beside the HCA pass,
+// which hides it: there the second read of K has to cost more than the step,
+// from about 64 MiB of K (48 for short chunks).  One read / two, time ratio by
+// HCA chunk, row groups a CSA chunk (g) and items, 8 heads and 64:
+//   32 KiB: bf16 D64 g1 of 32, 128, 192, 256 1.06, 1.04, 1.03, 1.00, g2 .95, .94,
+//   .93, .88; f32 D64 g1 .97 of 16 to 128; D256 bf16 .92-.97;
+//   64 KiB: bf16 D64 g1 of 64, 128, 256, 512 1.26, 1.16, 1.04, .87, g2 1.07, .96,
+//   .93, .78, g4 1.02, 1.01, .94, .80; bf16 D256 g2 of 64, 128, 192, 256 1.08, .99,
+//   .99, .95, g4 1.10, 1.03, 1.01, .97, g8 1.06, .98, .97, .94; f32 D64 g1 1.09,
+//   1.06, .98, .93, g2 .98, .89; f32 D128 .95-1.02 of 16 to 128; f32 D256 of 64,
+//   128 1.07, .97;
+//   128 KiB: bf16 D64 g1 of 128, 256, 512 1.40, 1.15, .84, g2 1.15, .95, .79, g4
+//   1.08, .93; bf16 D256 g2 of 128, 192, 256 1.15, 1.12, .95, g8 1.05, .99, .92; f32
+//   D64 g1 of 128, 192, 256 1.15, 1.05, .96, g2 of 32, 64 1.12, .97; f32 D128 g4
+//   of 64, 128 1.07, .98; f32 D256 1.10, .98;
+//   512 KiB: f32 D256 of 64, 1024 1.06, .71;
+//   bf16 D128, 48 MiB of K in chunks of 16 KiB .95; of 64 KiB g1 1.05, g4 1.03; of
+//   128 KiB g1 1.23, g4 1.01; 64 MiB of 96 KiB g3 .97, 128 KiB g1 1.06, g4 .93; 79
+//   MiB of 64 KiB g1 .88.
+inline bool csa_hybrid_one_read(int64_t esz, int64_t head_dim, int64_t csa_chunk, int64_t hca_chunk, int64_t items) {
+  constexpr int64_t KiB = 1024, MiB = 1024 * 1024;
+  const int64_t bytes = hca_chunk * head_dim * esz, groups = csa_chunk * head_dim * esz / 4096;
+  if (bytes > 128 * KiB && items < 512) return false;
+  if (esz == 2 && head_dim == 128)
+    return items * bytes >= (bytes <= 16 * KiB ? 48 * MiB : groups <= 1 && bytes > 64 * KiB ? 80 * MiB : 64 * MiB);
   int64_t fewest = 1;
-  if (bytes > 128 * KiB)
-    fewest = 512;
-  else if (bytes > 64 * KiB)
-    fewest = esz == 4 ? 64 : head_dim == 64 ? 257 : 256;
-  else if (bytes > 32 * KiB && esz == 2 && head_dim == 64)
-    fewest = 128;
-  if (items < fewest) return false;
-  return esz == 4 || head_dim != 128 || items * bytes >= (int64_t{48} << 20);
+  if (bytes > 64 * KiB)
+    fewest = esz == 4 ? (groups <= 1 ? 256 : 128) : groups <= 1 ? 512 : groups >= 8 ? 192 : 256;
+  else if (bytes > 32 * KiB)
+    fewest = esz == 4 ? (groups <= 1 ? 192 : head_dim == 256 ? 128 : 1)
+                      : groups <= 1 ? 512 : head_dim == 64 || groups >= 8 ? 128 : 256;
+  else if (bytes > 16 * KiB && esz == 2 && groups <= 1)
+    fewest = 256;
+  return items >= fewest;
 }
 
 }  // namespace csahca

@@ -292,7 +292,7 @@ bool hybrid_one_read(int dtype, int64_t head_dim, int64_t csa_chunk, int64_t hca
   if (hca_chunk % csa_chunk != 0 || csa_chunk % (kHcaThreads * (16 / esz) / head_dim) != 0) return false;
   const int env = env_one_read();
   if (env >= 0) return env == 1;
-  return csa_hybrid_one_read(esz, head_dim, hca_chunk, items);
+  return csa_hybrid_one_read(esz, head_dim, csa_chunk, hca_chunk, items);
 }
 }  // namespace
 

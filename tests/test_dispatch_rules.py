@@ -15,8 +15,8 @@ extern "C" {
 int64_t split_tile(int64_t tile, int64_t total, int64_t bh, int64_t D, int64_t esz, int vec) {
   return csahca::csa_split_tile(tile, total, bh, D, esz, vec != 0);
 }
-int hybrid_one_read(int64_t esz, int64_t D, int64_t hca_chunk, int64_t items) {
-  return csahca::csa_hybrid_one_read(esz, D, hca_chunk, items);
+int hybrid_one_read(int64_t esz, int64_t D, int64_t chunk, int64_t hca_chunk, int64_t items) {
+  return csahca::csa_hybrid_one_read(esz, D, chunk, hca_chunk, items);
 }
 int select_topk_regs(int64_t C, int64_t k) { return csahca::csa_select_topk_regs(C, k); }
 int step_topk_regs(int64_t C, int64_t k, int64_t bh, int fine) {
@@ -37,7 +37,7 @@ def rules(tmp_path_factory):
     lib.split_tile.argtypes = [ctypes.c_int64] * 5 + [ctypes.c_int]
     lib.step_topk_regs.argtypes = [ctypes.c_int64] * 3 + [ctypes.c_int]
     lib.select_topk_regs.argtypes = [ctypes.c_int64] * 2
-    lib.hybrid_one_read.argtypes = [ctypes.c_int64] * 4
+    lib.hybrid_one_read.argtypes = [ctypes.c_int64] * 5
     return lib
 
 
@@ -148,27 +148,45 @@ def test_selection_op_takes_registers_up_to_192_chunks(rules, C, k, want):
     assert rules.select_topk_regs(C, k) == want
 
 
-@pytest.mark.parametrize("esz,D,hca_chunk,items,want", [
-    (2, 64, 256, 1, 1),         # 32 KiB an item
-    (2, 64, 512, 127, 0),       # 64 KiB: one read 7-9% slower
-    (2, 64, 512, 128, 1),
-    (2, 64, 1024, 256, 0),      # 128 KiB: 15-38% slower
-    (2, 64, 1024, 512, 1),
-    (2, 256, 128, 1, 1),
-    (2, 256, 256, 255, 0),      # 4-10% slower
-    (2, 256, 256, 256, 1),
-    (4, 64, 256, 1, 1),
-    (4, 64, 512, 63, 0),        # 6% slower
-    (4, 64, 512, 64, 1),
-    (4, 256, 256, 511, 0),      # more than 128 KiB
-    (4, 256, 256, 512, 1),
-    (2, 128, 256, 767, 0),      # 16-bit head_dim 128: from 48 MiB of K
-    (2, 128, 256, 768, 1),
-    (2, 128, 2048, 511, 0),
-    (4, 128, 64, 1, 1),
+@pytest.mark.parametrize("esz,D,chunk,hca_chunk,items,want", [
+    (2, 64, 32, 128, 1, 1),         # 16 KiB an item
+    (2, 64, 32, 256, 255, 0),       # 32 KiB, CSA chunks of one row group: 2-6% slower
+    (2, 64, 32, 256, 256, 1),
+    (2, 64, 64, 256, 1, 1),
+    (2, 64, 32, 512, 511, 0),       # 64 KiB: 4-27% slower
+    (2, 64, 64, 512, 127, 0),       # 7-9%
+    (2, 64, 64, 512, 128, 1),
+    (2, 64, 32, 1024, 511, 0),      # 128 KiB: 15-65%
+    (2, 64, 64, 1024, 255, 0),
+    (2, 64, 64, 1024, 256, 1),
+    (2, 256, 16, 64, 1, 1),
+    (2, 256, 32, 128, 255, 0),      # 1-10%
+    (2, 256, 32, 128, 256, 1),
+    (2, 256, 64, 128, 127, 0),
+    (2, 256, 64, 128, 128, 1),
+    (2, 256, 64, 256, 191, 0),
+    (2, 256, 64, 256, 192, 1),
+    (4, 64, 16, 128, 1, 1),
+    (4, 64, 16, 256, 191, 0),       # 4-9%
+    (4, 64, 32, 256, 1, 1),
+    (4, 64, 32, 512, 127, 0),       # 12%
+    (4, 64, 32, 512, 128, 1),
+    (4, 64, 16, 512, 255, 0),
+    (4, 128, 16, 128, 1, 1),
+    (4, 256, 16, 64, 127, 0),
+    (4, 256, 16, 64, 128, 1),
+    (4, 256, 64, 256, 511, 0),      # more than 128 KiB
+    (4, 256, 64, 256, 512, 1),
+    (2, 128, 64, 64, 3071, 0),      # 16-bit head_dim 128, 16 KiB: from 48 MiB of K
+    (2, 128, 64, 64, 3072, 1),
+    (2, 128, 64, 256, 1023, 0),     # 64 KiB: from 64 MiB (3% slower at 48)
+    (2, 128, 64, 256, 1024, 1),
+    (2, 128, 16, 512, 639, 0),      # 128 KiB, one row group: 6% slower at 64
+    (2, 128, 16, 512, 640, 1),
+    (2, 128, 64, 2048, 511, 0),
 ])
-def test_hybrid_reads_k_once_where_wavefronts_are_many(rules, esz, D, hca_chunk, items, want):
-    assert rules.hybrid_one_read(esz, D, hca_chunk, items) == want
+def test_hybrid_reads_k_once_where_wavefronts_are_many(rules, esz, D, chunk, hca_chunk, items, want):
+    assert rules.hybrid_one_read(esz, D, chunk, hca_chunk, items) == want
 
 
 def test_the_step_kernels_traffic_record_covers_every_source():
